@@ -48,6 +48,7 @@ SOURCES = [
     ("radix_sort.hip", "device"),
     ("cell_sort.hip", "device"),
     ("kernels.hip", "device"),
+    ("team.hip", "device"),
     ("twoscale.hip", "device"),
     ("sim.hip", "device"),
     ("neural.hip", "device"),

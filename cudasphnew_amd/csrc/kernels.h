@@ -69,5 +69,11 @@ void launch_surface(hipStream_t st, const StepBuffers& b, float cm_thresh, float
 void launch_export_positions(hipStream_t st, uint32_t n, const float4* pos, const float4* vel, const uint32_t* oid,
                              float4* out);
 void launch_force(hipStream_t st, const StepBuffers& b, int lanes, int block = 256);
+// The one-lane and hit-mask variants of a small particle set (team.hip):
+// sixteen lanes per particle, the same results bit for bit.  team_step:
+// whether this step's buffers take them, the same answer for both passes.
+bool team_step(const StepBuffers& b);
+void launch_density_team(hipStream_t st, const StepBuffers& b);
+void launch_force_team(hipStream_t st, const StepBuffers& b);
 
 }  // namespace sph

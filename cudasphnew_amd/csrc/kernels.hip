@@ -15,23 +15,11 @@
 //   original-id order) -> density -> force + integrate + collision + next
 //   key.
 #include "kernels.h"
+#include "step_device.h"
 
 namespace sph {
 
 namespace {
-
-constexpr int kBlock = 256;
-
-inline unsigned blocks_for(uint32_t n, int block) { return (n + block - 1) / block; }
-
-// Scene record of a slot.  ONE (a single scene, every handle's case): index
-// 0, a uniform address, so the record's fields are scalar loads; else the
-// binary search over the scene begins, per lane (vector loads).
-template <bool ONE>
-__device__ __forceinline__ const DevScene& scene_for(const DevScene* __restrict__ scenes,
-                                                     const uint32_t* __restrict__ begins, int nscenes, uint32_t s) {
-    return ONE ? scenes[0] : scenes[scene_of(begins, nscenes, s)];
-}
 
 // Slot of a lane in the hit-mask kernels.  ONE: consecutive slots, lanes
 // past the end repeat the last slot (not live).  Batch: the work list holds
@@ -175,209 +163,6 @@ __global__ __launch_bounds__(kBlock) void k_export_positions(uint32_t n, const f
     out[oid[i]] = make_float4(p.x, p.y, p.z, vel[i].w);
 }
 
-// Contiguous slot run of the cells [i0, i1] of one x-row (cells of a row
-// have consecutive keys, so their particles are consecutive slots).
-__device__ __forceinline__ void row_run(const int2* __restrict__ range, uint32_t rowbase, int i0, int i1, int& b,
-                                        int& e) {
-    b = 0x7fffffff;
-    e = -1;
-    for (int i = i0; i <= i1; ++i) {
-        int2 r = range[rowbase + (uint32_t)i];
-        if (r.x >= 0) {
-            b = min(b, r.x);
-            e = max(e, r.y);
-        }
-    }
-}
-
-// Neighbour range of a particle on the coarse grid (compute_grid_coordinate,
-// cu:1238-1258) and the nine x-row runs of it.
-struct Rows {
-    int lx, hx, ly, hy, lz, hz;
-};
-
-__device__ __forceinline__ Rows neighbour_rows(const DevScene& S, float4 xi) {
-    const float h = S.h;
-    Rows r;
-    r.lx = range_coord(xi.x, -h, S.ox, S.cell, S.nx); r.hx = range_coord(xi.x, h, S.ox, S.cell, S.nx);
-    r.ly = range_coord(xi.y, -h, S.oy, S.cell, S.ny); r.hy = range_coord(xi.y, h, S.oy, S.cell, S.ny);
-    r.lz = range_coord(xi.z, -h, S.oz, S.cell, S.nz); r.hz = range_coord(xi.z, h, S.oz, S.cell, S.nz);
-    return r;
-}
-
-// Slot run of row (dk, dj) of the 3x3 row set; empty when the row is outside
-// the clamped range (e.g. at the grid edge, or the reference's wrapped upper
-// coordinate).
-__device__ __forceinline__ void row_slots(const int2* __restrict__ range, const DevScene& S, const Rows& R, int dk,
-                                          int dj, float4 xi, int& b, int& e) {
-    const int k = R.lz + dk, j = R.ly + dj;
-    b = 0;
-    e = 0;
-    if (k > R.hz || j > R.hy) return;
-    // a row whose y-z cell rectangle is farther than h from the particle
-    // holds no neighbour (its candidates would add exact zeros); the 1e-5
-    // margin covers the rounding of the cell bounds and of the keys
-    const float y0 = S.oy + (float)j * S.cell, z0 = S.oz + (float)k * S.cell;
-    const float dy = fmaxf(fmaxf(y0 - xi.y, xi.y - (y0 + S.cell)), 0.0f);
-    const float dz = fmaxf(fmaxf(z0 - xi.z, xi.z - (z0 + S.cell)), 0.0f);
-    if ((dy * dy + dz * dz) * 0.99999f > S.h2) return;
-    uint32_t rowbase = S.cell_offset + (uint32_t)(S.nx * (S.ny * k + j));
-    row_run(range, rowbase, R.lx, R.hx, b, e);
-    if (e < b) { b = 0; e = 0; }
-}
-
-// Pair terms of the acceleration (cu:1486-1555) accumulated without the
-// constant factors: m, gradSpiky, mu, laplVisc, gradPoly6, laplPoly6 are
-// applied once in force_finish.
-struct PairSums {
-    float fpx, fpy, fpz, fvx, fvy, fvz, cgx, cgy, cgz, cl;
-};
-
-// GUARD: the caller has not tested r2 > 0; a pair at distance 0 then adds
-// exact zeros (inverse distance and 1/rho_j taken as 0).
-template <bool GUARD = false>
-__device__ __forceinline__ void pair_terms(PairSums& a, float4 xi, float4 vi, float rhoi, float Ai, float h, float h2,
-                                           float stiff, float kr0, float4 xj, float4 vj) {
-    float dx = xi.x - xj.x, dy = xi.y - xj.y, dz = xi.z - xj.z;
-    float r2 = dx * dx + dy * dy + dz * dz;
-    float inv_r = __builtin_amdgcn_rsqf(r2);
-    float invj = __builtin_amdgcn_rcpf(vj.w);
-    if (GUARD) {
-        const bool ok = r2 > 0.0f;
-        inv_r = ok ? inv_r : 0.0f;
-        invj = ok ? invj : 0.0f;
-    }
-    float rn = r2 * inv_r;
-    float pj = stiff * vj.w - kr0;
-    float hr = h - rn;
-    float qd = h2 - r2;
-    float cp = (Ai + rhoi * pj * invj * invj) * hr * hr * inv_r;
-    a.fpx += cp * dx; a.fpy += cp * dy; a.fpz += cp * dz;
-    float wv = invj * hr;
-    a.fvx += wv * (vj.x - vi.x); a.fvy += wv * (vj.y - vi.y); a.fvz += wv * (vj.z - vi.z);
-    float wc = invj * qd * qd;
-    a.cgx += wc * dx; a.cgy += wc * dy; a.cgz += wc * dz;
-    a.cl += invj * qd * (3.0f * h2 - 7.0f * r2);
-}
-
-// Wall penalty + wall viscosity or surface tension (cu:407-466), a = F/rho - g
-// (cu:470-473), symplectic Euler (integrate_euler, cu:632-665), the
-// grid-driven collision response (collision_handling, cu:742-834) and the
-// next step's cell key; writes the next storage order (this step's sorted
-// order).
-__device__ __forceinline__ void force_finish(const DevScene& S, uint32_t s, float4 xi, float4 vi, const PairSums& a,
-                                             const float4* __restrict__ grid4, const float* __restrict__ gridd,
-                                             const uint32_t* __restrict__ oid_b, const uint8_t* __restrict__ state_b,
-                                             float4* __restrict__ acc, float4* __restrict__ pos_out,
-                                             float4* __restrict__ vel_out, uint32_t* __restrict__ oid_out,
-                                             uint8_t* __restrict__ state_out, uint32_t* __restrict__ key_out,
-                                             uint32_t* __restrict__ status, const NeuralRefs& nr) {
-    const float rhoi = vi.w;
-    const float cpf = -S.mass * S.grad_spiky, cvf = S.mu * S.mass * S.lapl_visc;
-    float Fx = cvf * a.fvx + cpf * a.fpx, Fy = cvf * a.fvy + cpf * a.fpy, Fz = cvf * a.fvz + cpf * a.fpz;
-    const int wm = wall_mode(nr, s);
-    float tx, ty, tz;
-    texel_coords(S, xi.x, xi.y, xi.z, tx, ty, tz);
-    // distance and wall viscosity from the grid (the wall-term switch
-    // distWall < r0 and the penalty magnitude need its exact values); a cell
-    // far from every surface takes no wall term and no lookup; with the
-    // learned source the penalty and collision normals come from the
-    // network's gradient instead of central differences of the grid
-    float distWall = S.r0, wvisc = 0.0f;
-    float4 r1 = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    if (wm != kWallNone) {
-        float4 g = lerp3<float4>(grid4, S, tex_setup(S, tx, ty, tz));
-        distWall = -g.x;
-        wvisc = g.z;
-        if (wm == kWallNeural && nr.need[s]) r1 = nr.rec[s];   // central-difference gradient of the learned distance at x
-    }
-    // the network's normal exists where the density pass asked for it
-    const bool net_normal = wm == kWallNeural && nr.need[s];
-    if (distWall < S.r0) {
-        float coeff = rhoi / (S.dt * S.dt) * (S.r0 - distWall);
-        // normalized-coordinate gradient: learned source dD/dx times
-        // dx/du = L = dims / bscale per axis
-        float3 gn = net_normal ? make_float3(r1.x * ((float)S.bnx / S.bscale_x), r1.y * ((float)S.bny / S.bscale_y),
-                                             r1.z * ((float)S.bnz / S.bscale_z))
-                               : dist_grad_normalized(gridd, S, tx, ty, tz);
-        Fx -= coeff * gn.x + vi.x * wvisc;
-        Fy -= coeff * gn.y + vi.y * wvisc;
-        Fz -= coeff * gn.z + vi.z * wvisc;
-    } else {
-        float cm = S.mass * S.grad_poly6;
-        float gx = cm * a.cgx, gy = cm * a.cgy, gz = cm * a.cgz;
-        float gnorm = sqrtf(gx * gx + gy * gy + gz * gz);
-        if (gnorm > S.norm_thresh) {
-            float fc = S.sigma * (S.mass * S.lapl_poly6 * a.cl) / gnorm;
-            Fx -= fc * gx;
-            Fy -= fc * gy;
-            Fz -= fc * gz;
-        }
-    }
-    float ax = Fx / rhoi, ay = Fy / rhoi - S.gravity, az = Fz / rhoi;
-    acc[s] = make_float4(ax, ay, az, 0.0f);
-    float vx = vi.x + S.dt * ax, vy = vi.y + S.dt * ay, vz = vi.z + S.dt * az;
-    float px = xi.x + S.dt * vx, py = xi.y + S.dt * vy, pz = xi.z + S.dt * vz;
-    if (S.collision && wm != kWallNone) {
-        float D;
-        float3 gw;
-        float cx, cy, cz;
-        texel_coords(S, px, py, pz, cx, cy, cz);
-        D = dist_at(gridd, S, cx, cy, cz);
-        if (D > 0.0f) {
-            if (net_normal) {
-                gw = make_float3(r1.x, r1.y, r1.z);   // learned source: its gradient at the old position
-            } else {
-                gw = dist_grad_normalized(gridd, S, cx, cy, cz);
-                // normalized-coordinate gradient -> world gradient: divide by L
-                gw.x *= S.bscale_x * (1.0f / (float)S.bnx);
-                gw.y *= S.bscale_y * (1.0f / (float)S.bny);
-                gw.z *= S.bscale_z * (1.0f / (float)S.bnz);
-            }
-        }
-        if (D > 0.0f) {
-            float gl = sqrtf(gw.x * gw.x + gw.y * gw.y + gw.z * gw.z);
-            if (gl > 0.0f) {
-                float nx_ = gw.x / gl, ny_ = gw.y / gl, nz_ = gw.z / gl;
-                float vn = sqrtf(vx * vx + vy * vy + vz * vz);
-                float dp = nx_ * vx + ny_ * vy + nz_ * vz;
-                float c = 1.0f;
-                if (S.restitution != 0.0f && vn > 0.0f) c += S.restitution * D / (S.dt * vn);
-                c *= dp;
-                vx -= c * nx_; vy -= c * ny_; vz -= c * nz_;
-                px -= D * nx_; py -= D * ny_; pz -= D * nz_;
-            }
-        }
-    }
-    uint32_t flags = 0;
-    uint32_t kk = cell_key(S, px, py, pz, flags);
-    if (!(isfinite(px) && isfinite(py) && isfinite(pz) && isfinite(vx) && isfinite(vy) && isfinite(vz)))
-        flags |= kStatusNonFinite;
-    if (flags) atomicOr(status, flags);
-    pos_out[s] = make_float4(px, py, pz, rhoi);
-    vel_out[s] = make_float4(vx, vy, vz, rhoi);
-    key_out[s] = kk;
-    oid_out[s] = oid_b[s];
-    if (state_out) state_out[s] = state_b[s];
-}
-
-__device__ __forceinline__ float wall_density(const DevScene& S, const float4* __restrict__ grid4, float4 xi,
-                                              const NeuralRefs& nr, uint32_t s) {
-    // the density pass flags the network's particles; it also starts their
-    // lists (the network pass appends after it)
-    if (s == 0 && nr.list_count)
-        for (int i = 0; i < nr.nscenes; ++i) nr.list_count[i] = 0u;
-    const int wm = wall_mode(nr, s);
-    if (wm == kWallNone) return 0.0f;
-    float tx, ty, tz;
-    texel_coords(S, xi.x, xi.y, xi.z, tx, ty, tz);
-    const float4 g = lerp3<float4>(grid4, S, tex_setup(S, tx, ty, tz));
-    // learned source: the force pass needs the network's normal exactly
-    // where the wall penalty acts (distWall = -D < r0)
-    if (wm == kWallNeural && nr.need) nr.need[s] = g.x > -S.r0;
-    return g.y;
-}
-
 // compute_particle_density_pressure (cu:196-256, 1385-1419), one thread per
 // particle.  Density goes to vel.w; pressure k(rho - rho0) is recomputed
 // where needed.
@@ -400,10 +185,7 @@ __global__ __launch_bounds__(B) void k_density(const float4* __restrict__ pos, f
             row_slots(range, S, R, dk, dj, xi, b, e);
 #pragma unroll 4
             for (int q = b; q < e; ++q) {
-                float4 xj = pos[q];
-                float dx = xj.x - xi.x, dy = xj.y - xi.y, dz = xj.z - xi.z;
-                float r2 = dx * dx + dy * dy + dz * dz;
-                float d = fmaxf(h2 - r2, 0.0f);
+                const float d = density_gap(xi, pos[q], h2);
                 sum += d * d * d;
             }
         }
@@ -444,7 +226,7 @@ __global__ __launch_bounds__(kBlock) void k_density_coop(const float4* __restric
                     for (int q = b + c; q < e; q += L) {
                         float4 xj = pos[q];
                         float dx = xj.x - xi.x, dy = xj.y - xi.y, dz = xj.z - xi.z;
-                        float r2 = dx * dx + dy * dy + dz * dz;
+                        float r2 = sq3(dx, dy, dz);
                         float d = fmaxf(h2 - r2, 0.0f);
                         sum += d * d * d;
                     }
@@ -498,7 +280,7 @@ __global__ __launch_bounds__(B) void k_force(
                 for (int t = 0; t < cnt; ++t) {
                     float4 xj = pos[base + t];
                     float dx = xi.x - xj.x, dy = xi.y - xj.y, dz = xi.z - xj.z;
-                    float r2 = dx * dx + dy * dy + dz * dz;
+                    float r2 = sq3(dx, dy, dz);
                     hits |= (uint64_t)(r2 <= h2 && r2 > 0.0f) << t;
                 }
                 while (hits) {
@@ -563,7 +345,7 @@ __global__ __launch_bounds__(kBlock) void k_force_coop(
                     if (q < e) {
                         float4 xj = pos[q];
                         float dx = xi.x - xj.x, dy = xi.y - xj.y, dz = xi.z - xj.z;
-                        float r2 = dx * dx + dy * dy + dz * dz;
+                        float r2 = sq3(dx, dy, dz);
                         hit = r2 <= h2 && r2 > 0.0f;
                     }
                     const uint64_t vote = __ballot(hit);
@@ -593,7 +375,7 @@ __global__ __launch_bounds__(kBlock) void k_force_coop(
                     for (int q = b; q < e; ++q) {
                         float4 xj = pos[q];
                         float dx = xi.x - xj.x, dy = xi.y - xj.y, dz = xi.z - xj.z;
-                        float r2 = dx * dx + dy * dy + dz * dz;
+                        float r2 = sq3(dx, dy, dz);
                         if (r2 <= h2 && r2 > 0.0f) pair_terms(a, xi, vi, rhoi, Ai, h, h2, S.stiff, kr0, xj, vel[q]);
                     }
                 }
@@ -650,22 +432,6 @@ __global__ __launch_bounds__(kBlock) void k_force_coop(
 // invert, drop the unused high part.
 __device__ __forceinline__ uint32_t near_bits(uint32_t far, int c) {
     return c > 0 ? __builtin_bitreverse32(~far) >> (32 - c) : 0u;
-}
-
-// One candidate of the density pass: poly6 sum and the "farther than h" bit.
-// d = h2 - dz^2 - dy^2 - dx^2 as a chain of three fused multiply-adds (one
-// instruction fewer than forming r^2 and subtracting it).  Each step rounds
-// an exact result, which keeps its sign (and an exact zero is +0), so d's
-// sign bit is set exactly when this d is negative, i.e. when the candidate's
-// poly6 term is zero: the bit is that "farther than h" bit and one funnel
-// shift per candidate builds the mask.
-__device__ __forceinline__ void density_candidate(float xjx, float xjy, float xjz, float4 xi, float h2, float& sum,
-                                                  uint32_t& far) {
-    float dx = xjx - xi.x, dy = xjy - xi.y, dz = xjz - xi.z;
-    float d = fmaf(-dx, dx, fmaf(-dy, dy, fmaf(-dz, dz, h2)));
-    far = __builtin_amdgcn_alignbit(far, __float_as_uint(d), 31);
-    d = fmaxf(d, 0.0f);
-    sum += d * d * d;
 }
 
 // The candidates [0, cnt) of one row run: adds their poly6 terms to sum and
@@ -960,7 +726,7 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(CAP <= 40 ? 5
                 for (int q = b; q < e; ++q) {
                     float4 xj = pos[q];
                     float dx = xi.x - xj.x, dy = xi.y - xj.y, dz = xi.z - xj.z;
-                    float r2 = dx * dx + dy * dy + dz * dz;
+                    float r2 = sq3(dx, dy, dz);
                     if (r2 <= h2 && r2 > 0.0f) pair_terms<false>(a, xi, vi, rhoi, Ai, h, h2, S.stiff, kr0, xj, vel[q]);
                 }
             }
@@ -992,7 +758,7 @@ __global__ __launch_bounds__(kBlock) void k_surface(const float4* __restrict__ p
             for (int q = b; q < e; ++q) {
                 const float4 xj = pos[q];
                 const float dx = xj.x - xi.x, dy = xj.y - xi.y, dz = xj.z - xi.z;
-                const float r2 = dx * dx + dy * dy + dz * dz;
+                const float r2 = sq3(dx, dy, dz);
                 if (r2 <= S.h2 && r2 > 0.0f) {
                     sx += dx;
                     sy += dy;
@@ -1096,6 +862,7 @@ static void launch_density_one_lane(hipStream_t st, const StepBuffers& b) {
 
 void launch_density(hipStream_t st, const StepBuffers& b, int lanes, int block) {
     const bool small = block == 128, one = b.nscenes == 1;
+    if ((b.masks || lanes == 1) && team_step(b)) return launch_density_team(st, b);
     if (b.masks) {
         if (small) one ? launch_density_masks<128, true>(st, b) : launch_density_masks<128, false>(st, b);
         else one ? launch_density_masks<kBlock, true>(st, b) : launch_density_masks<kBlock, false>(st, b);
@@ -1148,6 +915,7 @@ static void launch_force_masks(hipStream_t st, const StepBuffers& b, int cap) {
 
 void launch_force(hipStream_t st, const StepBuffers& b, int lanes, int block) {
     const bool small = block == 128, one = b.nscenes == 1;
+    if ((b.masks || lanes == 1) && team_step(b)) return launch_force_team(st, b);
     if (b.masks) {
         // lanes selects the LDS hit-list capacity of the hit-mask variant
         if (small) one ? launch_force_masks<128, true>(st, b, lanes) : launch_force_masks<128, false>(st, b, lanes);
