@@ -104,7 +104,15 @@ __device__ __forceinline__ f32x4 mfma(bf16x8 a, bf16x8 b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 
-__device__ __forceinline__ float sigmoid(float z) { return 1.0f / (1.0f + __expf(-z)); }
+// 1 / (1 + exp(-z)).  One Newton step on the hardware reciprocal of a number
+// in [1, 2^126] is the correctly rounded quotient (checked against 1.0f / d
+// over every mantissa of the binades), in half the division's operations; past
+// 2^126 (z < -87) the result stays at 2^-126.
+__device__ __forceinline__ float sigmoid(float z) {
+    const float d = fminf(1.0f + __expf(-z), 0x1p126f);
+    const float r = __builtin_amdgcn_rcpf(d);
+    return fmaf(fmaf(-d, r, 1.0f), r, r);
+}
 
 // sin(pi x) and cos(pi x): exact reduction to r = x - 2 rint(x/2) in
 // [-1, 1] (|x| < 2^22 here), then the hardware sine/cosine of r/2
@@ -244,21 +252,6 @@ __device__ __forceinline__ void store_dz(const f32x4 dz[4], int lane, int w, uin
     }
 }
 
-// dW^T[n_out rows of wave w][k_in tiles] += dZ^T . A over the 64 samples.
-template <int NC>
-__device__ __forceinline__ void weight_grad(const uint16_t* sdZT, const uint16_t* sAT, int lane, int w,
-                                            f32x4 acc[NC]) {
-#pragma unroll
-    for (int ks = 0; ks < kTile / 32; ++ks) {
-        bf16x8 a = frag_ld(sdZT + (16 * w + (lane & 15)) * kLds + 32 * ks + 8 * (lane >> 4));
-#pragma unroll
-        for (int c = 0; c < NC; ++c) {
-            bf16x8 b = frag_ld(sAT + (16 * c + (lane & 15)) * kLds + 32 * ks + 8 * (lane >> 4));
-            acc[c] = mfma(a, b, acc[c]);
-        }
-    }
-}
-
 // Sum over the 16 lanes that share lane/16 (one sample row group).
 __device__ __forceinline__ float row_sum16(float v) {
     v += __shfl_xor(v, 1, 64);
@@ -268,166 +261,347 @@ __device__ __forceinline__ float row_sum16(float v) {
     return v;
 }
 
-// Sum over the four lane groups (lane/16) with the same lane%16.
-__device__ __forceinline__ float col_sum4(float v) {
-    v += __shfl_xor(v, 16, 64);
-    v += __shfl_xor(v, 32, 64);
+// ---- training ----------------------------------------------------------------
+//
+// A workgroup works tiles of 128 samples, wavefront w owning samples
+// 16w .. 16w + 15 of the row-parallel products.  Every product is taken with
+// the sample on the columns, D[n][s] = sum_k W[n][k] X[k][s], so that a lane
+// holds four consecutive outputs of one sample: activations and dz go to LDS
+// as one 8-byte store per 16 outputs, sample-major, and a wavefront's forward
+// and backward chain reads only what it wrote itself (no barrier).  The
+// weight gradients, sums over the tile's samples, read the same arrays
+// transposed on the way out of LDS (ds_read_b64_tr_b16): one barrier before
+// them, one after.  Before, both layouts were stored, 2 bytes a store, with
+// a barrier at each of the six layer steps.
+//
+// A forward fragment is the A operand here and was the B operand of the
+// transposed product: the same products summed in the same order.
+
+constexpr int kLdsX = kK1 + 8;          // row stride of the feature tile
+// Partial gradient vectors: the parameters' sections, the three matrices
+// inside theirs in accumulator order (16 x 16 tile by tile, lane by lane,
+// four consecutive outputs per lane), so that a block stores them as whole
+// cache lines; padded to 16 bytes.
+constexpr int kPartStride = (kParams + 3) / 4 * 4;
+static_assert(ob1 % 4 == 0 && oW2 % 4 == 0 && ob2 % 4 == 0 && oW3 % 4 == 0 && ob3 % 4 == 0 && ow4 % 4 == 0 &&
+                  ob4 % 4 == 0,
+              "sections are read four values at a time");
+
+__device__ __forceinline__ uint2 pack4(float a, float b, float c, float d) {
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    const f32x2 lo = {a, b}, hi = {c, d};
+    return make_uint2(__builtin_bit_cast(uint32_t, __builtin_convertvector(lo, bf16x2)),
+                      __builtin_bit_cast(uint32_t, __builtin_convertvector(hi, bf16x2)));
+}
+
+// LDS written by lanes of a wavefront and read by its other lanes.
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Fragment of a sample-major LDS tile read transposed: element e of lane l is
+// tile[row0 + 8 (l / 16) + e][col0 + l % 16].  ds_read_b64_tr_b16 works on 16
+// lanes: lane i supplies four columns 4 (i % 4) of row i / 4 and receives
+// column i of the four rows.
+__device__ __forceinline__ bf16x8 frag_tr(const uint16_t* tile, int stride, int row0, int col0, int lane) {
+    typedef short s16x4 __attribute__((ext_vector_type(4)));
+    typedef __attribute__((address_space(3))) s16x4* lds_ptr;
+    const uint16_t* p = tile + (row0 + 8 * (lane >> 4) + ((lane & 15) >> 2)) * stride + col0 + 4 * (lane & 3);
+    const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(p));
+    const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(p + 4 * stride));
+    typedef short s16x8 __attribute__((ext_vector_type(8)));
+    const s16x8 v = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+    return __builtin_bit_cast(bf16x8, v);
+}
+
+// acc[c] (outputs 16c ..) += W . X for the wavefront's 16 samples, both from
+// LDS: the 64 x 64 matrix W[n][k] as stored (BACK = false), or transposed, for
+// the back-propagation through it (BACK = true).
+template <bool BACK>
+__device__ __forceinline__ void w_x_cols(const uint16_t* sW, const uint16_t* sX, int lane, f32x4 acc[4]) {
+#pragma unroll
+    for (int c = 0; c < 4; ++c) acc[c] = f32x4{0, 0, 0, 0};
+#pragma unroll
+    for (int ks = 0; ks < kH / 32; ++ks) {
+        const bf16x8 x = frag_ld(sX + (lane & 15) * kLds + 32 * ks + 8 * (lane >> 4));
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+            acc[c] = mfma(BACK ? frag_tr(sW, kLds, 32 * ks, 16 * c, lane)
+                               : frag_ld(sW + (16 * c + (lane & 15)) * kLds + 32 * ks + 8 * (lane >> 4)),
+                          x, acc[c]);
+    }
+}
+
+// ROWS rows of K BF16 values into LDS rows of LD.
+template <int ROWS, int K, int LD>
+__device__ __forceinline__ void stage(const uint16_t* __restrict__ W, uint16_t* sW, int threads) {
+    for (int i = threadIdx.x; i < ROWS * K / 8; i += threads) {
+        const int r = i / (K / 8), q = i % (K / 8);
+        *reinterpret_cast<uint4*>(sW + r * LD + 8 * q) = *reinterpret_cast<const uint4*>(W + 8 * i);
+    }
+}
+
+// Features k0 .. k0 + 7, k0 = 8 (4 ks + lane / 16), of normalized coordinates
+// u, packed as BF16.
+__device__ __forceinline__ uint4 feature_frag(const NetView& net, const float u[3], int ks, int lane) {
+    // features f0..f0+7 (f0 = 8q) use the (sin, cos) pairs
+    // m = 4q - 2 .. 4q + 2 (pair m = 3k + a: features 3 + 2m, 4 + 2m)
+    const int q = 4 * ks + (lane >> 4), f0 = 8 * q;
+    float ps[5], pc[5];
+#pragma unroll
+    for (int t = 0; t < 5; ++t) {
+        const int m = 4 * q - 2 + t;
+        ps[t] = pc[t] = 0.0f;
+        if (m >= 0 && m < 3 * kFreqs) sincospi_hw(net.freq[m / 3] * u[m % 3], ps[t], pc[t]);
+    }
+    float v[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const int f = f0 + j, t = (j + 1) >> 1;
+        v[j] = f < 3 ? u[f < 3 ? f : 0] : (f >= kFeat ? 0.0f : ((j & 1) ? ps[t] : pc[t]));
+    }
+    const uint2 a = pack4(v[0], v[1], v[2], v[3]), b = pack4(v[4], v[5], v[6], v[7]);
+    return make_uint4(a.x, a.y, b.x, b.y);
+}
+
+// Bias + SiLU of a layer's outputs (acc[c][j] = output 16c + 4 (lane / 16) + j
+// of sample lane % 16); the activations replace acc, silu'(z) goes to dact and
+// the BF16 activations to the sample's LDS row (if any).
+__device__ __forceinline__ void silu_cols(const float* __restrict__ bias, f32x4 acc[4], f32x4 dact[4], int lane,
+                                          uint16_t* row) {
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        const int n = 16 * c + 4 * (lane >> 4);
+        const float4 b = *reinterpret_cast<const float4*>(bias + n);
+        const float bn[4] = {b.x, b.y, b.z, b.w};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const float z = acc[c][j] + bn[j];
+            const float sg = sigmoid(z);
+            acc[c][j] = z * sg;
+            dact[c][j] = sg * (1.0f + z * (1.0f - sg));
+        }
+        if (row) *reinterpret_cast<uint2*>(row + n) = pack4(acc[c][0], acc[c][1], acc[c][2], acc[c][3]);
+    }
+}
+
+__device__ __forceinline__ void store_cols(const f32x4 v[4], int lane, uint16_t* row) {
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+        *reinterpret_cast<uint2*>(row + 16 * c + 4 * (lane >> 4)) = pack4(v[c][0], v[c][1], v[c][2], v[c][3]);
+}
+
+// Lane permutations inside 16 lanes, one VALU operation each (DPP).
+template <int CTRL>
+__device__ __forceinline__ float dpp(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, true));
+}
+constexpr int kDppXor1 = 0xB1, kDppXor3 = 0x1B, kDppXor7 = 0x141, kDppXor15 = 0x140;   // lane ^ 1, 3, 7, 15
+
+// Sum of a lane's value over the 16 lanes of its lane / 16 group.
+__device__ __forceinline__ float sum16(float v) {
+    v += dpp<kDppXor1>(v);
+    v += dpp<kDppXor3>(v);
+    v += dpp<kDppXor7>(v);
+    v += dpp<kDppXor15>(v);
     return v;
+}
+
+// Sums over the 16 lanes of a lane / 16 group of the 16 values v[c][j]: lane
+// l % 16 = 4c + j returns that of v[c][j].  Each step hands half of the
+// values left to the lane that keeps them (45 operations for 16 sums).
+template <int CTRL, int N>
+__device__ __forceinline__ void halve(float* v, bool upper) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        const float keep = upper ? v[i + N] : v[i], give = upper ? v[i] : v[i + N];
+        v[i] = keep + dpp<CTRL>(give);
+    }
+}
+
+__device__ __forceinline__ float scatter_sum16(const f32x4 a[4], int lane) {
+    float v[16];
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[4 * c + j] = a[c][j];
+    halve<kDppXor15, 8>(v, lane & 8);
+    halve<kDppXor7, 4>(v, lane & 4);
+    halve<kDppXor3, 2>(v, lane & 2);
+    halve<kDppXor1, 1>(v, lane & 1);
+    return v[0];
 }
 
 // One training pass over `batch` samples starting at `first` (wrapping at
 // n): forward, loss, backward; each block accumulates the gradient of its
 // tiles in registers and writes one partial gradient vector.
-__global__ __launch_bounds__(kThreads) void k_mlp_train(const float4* __restrict__ samples, uint32_t n,
-                                                        uint32_t first, uint32_t batch, NetView net,
-                                                        float* __restrict__ partial,
-                                                        float* __restrict__ loss_partial) {
-    __shared__ __align__(16) uint16_t sA0T[kK1 * kLds];
-    __shared__ __align__(16) uint16_t sA1[kTile * kLds], sA1T[kH * kLds];
-    __shared__ __align__(16) uint16_t sA2[kTile * kLds], sA2T[kH * kLds];
-    __shared__ __align__(16) uint16_t sdZ[kTile * kLds], sdZT[kH * kLds];
-    __shared__ float sred[4][4 * kH + 4];
+//
+// What bounds it: the latency of its chain of layers at two wavefronts a SIMD
+// (the tile's five arrays and the weights fill the LDS), then the VALU work
+// of features and activations.  128-sample tiles (eight wavefronts) against
+// 64-sample ones (four): 22.4 / 26.3 us a training step at batch 16,384, 15.8
+// / 15.7 at 64.  With the weights read from L2 for every tile instead of once
+// into LDS the kernel takes 45 us instead of 29 at batch 65,536.  Before this
+// layout: 80 us there, and 36 us for the sum of 512 partial vectors stored 4
+// bytes at a time (6.5 now); a training step 99.7 -> 36.2 us at 65,536,
+// 42.6 -> 22.4 at 16,384, 27.4 -> 15.8 at 64.
+constexpr int kTrainWaves = 8;
+constexpr int kTrainTile = 16 * kTrainWaves;
 
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+__global__ __launch_bounds__(64 * kTrainWaves) void k_mlp_train(const float4* __restrict__ samples, uint32_t n,
+                                                                uint32_t first, uint32_t batch, NetView net,
+                                                                float* __restrict__ partial,
+                                                                float* __restrict__ loss_partial) {
+    constexpr int NW = kTrainWaves, T = kTrainTile;
+    constexpr int C1 = 4, C2 = 2;   // accumulator tiles of a wavefront: half of a matrix's columns
+    __shared__ __align__(16) uint16_t sX[T * kLdsX];
+    __shared__ __align__(16) uint16_t sA[2][T * kLds];     // activations of layers 1, 2
+    __shared__ __align__(16) uint16_t sD[3][T * kLds];     // dz of layers 1, 2, 3
+    __shared__ __align__(16) uint16_t sW1[kH * kLdsX], sW2[kH * kLds], sW3[kH * kLds];   // [n][k]
+
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, l15 = lane & 15, g4 = 4 * (lane >> 4);
+    const int nb = w & 3, half = w >> 2;                   // output block and half of the weight gradients
+    const int row = 16 * w + l15;                          // this lane's sample of the tile
     const float* th = net.theta;
     const float gscale = 2.0f / (float)batch;
 
-    f32x4 gW1[8], gW2[4], gW3[4];
+    f32x4 gW1[C1], gW2[C2], gW3[C2];
 #pragma unroll
-    for (int c = 0; c < 8; ++c) gW1[c] = f32x4{0, 0, 0, 0};
+    for (int c = 0; c < C1; ++c) gW1[c] = f32x4{0, 0, 0, 0};
 #pragma unroll
-    for (int c = 0; c < 4; ++c) gW2[c] = gW3[c] = f32x4{0, 0, 0, 0};
-    float gb1[4] = {0, 0, 0, 0}, gb2[4] = {0, 0, 0, 0}, gb3[4] = {0, 0, 0, 0}, gw4[4] = {0, 0, 0, 0};
-    float gb4 = 0.0f, lsum = 0.0f;
-    float w4n[4];
-#pragma unroll
-    for (int c = 0; c < 4; ++c) w4n[c] = th[ow4 + 16 * c + (lane & 15)];
+    for (int c = 0; c < C2; ++c) gW2[c] = gW3[c] = f32x4{0, 0, 0, 0};
+    // bias and output-layer gradients of output 16 (l15 / 4) + g4 + l15 % 4
+    float gb1 = 0.0f, gb2 = 0.0f, gb3 = 0.0f, gw4 = 0.0f, gb4 = 0.0f, lsum = 0.0f;
     const float b4 = th[ob4];
 
-    const uint32_t ntiles = batch / kTile;
+    stage<kH, kK1, kLdsX>(net.w.W1T, sW1, 64 * NW);
+    stage<kH, kH, kLds>(net.w.W2T, sW2, 64 * NW);
+    stage<kH, kH, kLds>(net.w.W3T, sW3, 64 * NW);
+    __syncthreads();
+
+    const uint32_t ntiles = (batch + T - 1) / T;
     for (uint32_t t = blockIdx.x; t < ntiles; t += gridDim.x) {
         // ---- forward ----
-        const uint32_t sidx = (first + t * kTile + 16 * w + (lane & 15)) % n;
-        const float4 smp = samples[sidx];
+        const uint32_t pos = t * T + (uint32_t)row;
+        const bool live = pos < batch;                     // the last tile may be half full
+        const float4 smp = samples[(first + (live ? pos : 0u)) % n];
         float u[3];
         normalized(net, smp.x, smp.y, smp.z, u);
         f32x4 acc[4], D1[4], D2[4], D3[4];
 #pragma unroll
         for (int c = 0; c < 4; ++c) acc[c] = f32x4{0, 0, 0, 0};
-        input_layer(net, u, lane, w, acc, sA0T);
-        activate(th + ob1, acc, D1, lane, w, sA1, sA1T);
-        __syncthreads();
 #pragma unroll
-        for (int c = 0; c < 4; ++c) acc[c] = f32x4{0, 0, 0, 0};
-        rows_x_wt<kH, 4>(sA1, net.w.W2T, lane, w, acc);
-        activate(th + ob2, acc, D2, lane, w, sA2, sA2T);
-        __syncthreads();
+        for (int ks = 0; ks < kK1 / 32; ++ks) {
+            const uint4 pk = feature_frag(net, u, ks, lane);
+            *reinterpret_cast<uint4*>(sX + row * kLdsX + 32 * ks + 8 * (lane >> 4)) = pk;
+            const bf16x8 x = __builtin_bit_cast(bf16x8, pk);
 #pragma unroll
-        for (int c = 0; c < 4; ++c) acc[c] = f32x4{0, 0, 0, 0};
-        rows_x_wt<kH, 4>(sA2, net.w.W3T, lane, w, acc);
-        float a3[16];
-        activate(th + ob3, acc, D3, lane, w, nullptr, nullptr, a3);
-        // ---- output layer and loss (rows s_j = 16w + 4(lane/16) + j) ----
-        float g[4];
+            for (int c = 0; c < 4; ++c)
+                acc[c] = mfma(frag_ld(sW1 + (16 * c + l15) * kLdsX + 32 * ks + 8 * (lane >> 4)), x, acc[c]);
+        }
+        silu_cols(th + ob1, acc, D1, lane, sA[0] + row * kLds);
+        wave_sync();
+        w_x_cols<false>(sW2, sA[0] + 16 * w * kLds, lane, acc);
+        silu_cols(th + ob2, acc, D2, lane, sA[1] + row * kLds);
+        wave_sync();
+        w_x_cols<false>(sW3, sA[1] + 16 * w * kLds, lane, acc);
+        silu_cols(th + ob3, acc, D3, lane, nullptr);
+        // ---- output layer and loss ----
+        f32x4 p = f32x4{0, 0, 0, 0}, w4[4];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            float part = 0.0f;
+        for (int c = 0; c < 4; ++c) {
+            w4[c] = *reinterpret_cast<const f32x4*>(th + ow4 + 16 * c + g4);
 #pragma unroll
-            for (int c = 0; c < 4; ++c) part += a3[4 * c + j] * w4n[c];
-            float y = row_sum16(part) + b4;
-            // target of row s_j: held by lane 16*(s_j%16 / 16)... fetch it
-            // from the lane that loaded that sample (lane%16 == row in tile)
-            int row = 4 * (lane >> 4) + j;   // row within the wave's 16
-            float d_true = __shfl(smp.w, row, 64);
-            float e = y - target_of(net, d_true);
-            g[j] = gscale * e;
-            if ((lane & 15) == 0) lsum += e * e;
+            for (int j = 0; j < 4; ++j) p[j] += acc[c][j] * w4[c][j];
+        }
+        float y = (p[0] + p[1]) + (p[2] + p[3]);
+        y += __shfl_xor(y, 16, 64);
+        y += __shfl_xor(y, 32, 64);
+        const float e = live ? (y + b4) - target_of(net, smp.w) : 0.0f;
+        const float g = gscale * e;
+        if (lane < 16) {
+            lsum += e * e;
+            gb4 += g;
         }
         f32x4 dz[4];
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
+        for (int c = 0; c < 4; ++c)
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                gw4[c] += g[j] * a3[4 * c + j];
-                float v = g[j] * w4n[c] * D3[c][j];
-                dz[c][j] = v;
-                gb3[c] += v;
+                dz[c][j] = g * w4[c][j] * D3[c][j];
+                acc[c][j] *= g;
             }
+        gw4 += scatter_sum16(acc, lane);
+        gb3 += scatter_sum16(dz, lane);
+        store_cols(dz, lane, sD[2] + row * kLds);
+        wave_sync();
+        // ---- back-propagation to layers 2 and 1 ----
+        w_x_cols<true>(sW3, sD[2] + 16 * w * kLds, lane, acc);
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) dz[c][j] = acc[c][j] * D2[c][j];
+        gb2 += scatter_sum16(dz, lane);
+        store_cols(dz, lane, sD[1] + row * kLds);
+        wave_sync();
+        w_x_cols<true>(sW2, sD[1] + 16 * w * kLds, lane, acc);
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) dz[c][j] = acc[c][j] * D1[c][j];
+        gb1 += scatter_sum16(dz, lane);
+        store_cols(dz, lane, sD[0] + row * kLds);
+        __syncthreads();
+        // ---- weight gradients: dW^T[n][k] = sum over the tile's samples ----
+#pragma unroll
+        for (int ks = 0; ks < T / 32; ++ks) {
+            const bf16x8 d3 = frag_tr(sD[2], kLds, 32 * ks, 16 * nb, lane);
+            const bf16x8 d2 = frag_tr(sD[1], kLds, 32 * ks, 16 * nb, lane);
+            const bf16x8 d1 = frag_tr(sD[0], kLds, 32 * ks, 16 * nb, lane);
+#pragma unroll
+            for (int c = 0; c < C2; ++c) {
+                gW3[c] = mfma(d3, frag_tr(sA[1], kLds, 32 * ks, 16 * (C2 * half + c), lane), gW3[c]);
+                gW2[c] = mfma(d2, frag_tr(sA[0], kLds, 32 * ks, 16 * (C2 * half + c), lane), gW2[c]);
+            }
+#pragma unroll
+            for (int c = 0; c < C1; ++c)
+                gW1[c] = mfma(d1, frag_tr(sX, kLdsX, 32 * ks, 16 * (C1 * half + c), lane), gW1[c]);
         }
-        if ((lane & 15) == 0) gb4 += g[0] + g[1] + g[2] + g[3];
-        store_dz(dz, lane, w, sdZ, sdZT);
-        __syncthreads();
-        // ---- layer 3 gradient, back-propagate to layer 2 ----
-        weight_grad<4>(sdZT, sA2T, lane, w, gW3);
-#pragma unroll
-        for (int c = 0; c < 4; ++c) acc[c] = f32x4{0, 0, 0, 0};
-        rows_x_wt<kH, 4>(sdZ, net.w.W3, lane, w, acc);
-        __syncthreads();
-#pragma unroll
-        for (int c = 0; c < 4; ++c)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                dz[c][j] = acc[c][j] * D2[c][j];
-                gb2[c] += dz[c][j];
-            }
-        store_dz(dz, lane, w, sdZ, sdZT);
-        __syncthreads();
-        weight_grad<4>(sdZT, sA1T, lane, w, gW2);
-#pragma unroll
-        for (int c = 0; c < 4; ++c) acc[c] = f32x4{0, 0, 0, 0};
-        rows_x_wt<kH, 4>(sdZ, net.w.W2, lane, w, acc);
-        __syncthreads();
-#pragma unroll
-        for (int c = 0; c < 4; ++c)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                dz[c][j] = acc[c][j] * D1[c][j];
-                gb1[c] += dz[c][j];
-            }
-        store_dz(dz, lane, w, sdZ, sdZT);
-        __syncthreads();
-        weight_grad<8>(sdZT, sA0T, lane, w, gW1);
-        __syncthreads();   // LDS tiles are rewritten by the next tile
+        __syncthreads();   // the tiles are rewritten by the next one
     }
 
-    // ---- write this block's partial gradient ----
-    float* out = partial + (size_t)blockIdx.x * kParams;
-    // dW^T accumulators: row n_out = 16w + 4(lane/16) + j, col k_in = 16c + lane%16
+    // ---- this block's partial gradient ----
+    float* out = partial + (size_t)blockIdx.x * kPartStride;
 #pragma unroll
-    for (int c = 0; c < 8; ++c)
+    for (int c = 0; c < C1; ++c)
+        *reinterpret_cast<f32x4*>(out + oW1 + ((nb * 8 + C1 * half + c) * 64 + lane) * 4) = gW1[c];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            int no = 16 * w + 4 * (lane >> 4) + j, ki = 16 * c + (lane & 15);
-            out[oW1 + ki * kH + no] = gW1[c][j];
-        }
-#pragma unroll
-    for (int c = 0; c < 4; ++c)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            int no = 16 * w + 4 * (lane >> 4) + j, ki = 16 * c + (lane & 15);
-            out[oW2 + ki * kH + no] = gW2[c][j];
-            out[oW3 + ki * kH + no] = gW3[c][j];
-        }
-    // column sums: reduce over lane groups, then over the four waves
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-        float v1 = col_sum4(gb1[c]), v2 = col_sum4(gb2[c]), v3 = col_sum4(gb3[c]), v4 = col_sum4(gw4[c]);
-        if (lane < 16) {
-            int n = 16 * c + lane;
-            sred[w][n] = v1;
-            sred[w][kH + n] = v2;
-            sred[w][2 * kH + n] = v3;
-            sred[w][3 * kH + n] = v4;
-        }
+    for (int c = 0; c < C2; ++c) {
+        *reinterpret_cast<f32x4*>(out + oW2 + ((nb * 4 + C2 * half + c) * 64 + lane) * 4) = gW2[c];
+        *reinterpret_cast<f32x4*>(out + oW3 + ((nb * 4 + C2 * half + c) * 64 + lane) * 4) = gW3[c];
     }
-    float l4 = col_sum4(gb4), ls = col_sum4(lsum);
+    // the per-output sums: over the 16 samples of the lanes, then over the
+    // wavefronts (through the tiles' LDS, no longer read)
+    float(*sred)[4 * kH + 2] = reinterpret_cast<float(*)[4 * kH + 2]>(&sX[0]);
+    static_assert(sizeof(sX) >= sizeof(float) * NW * (4 * kH + 2), "reduction fits the feature tile");
+    const int o = 16 * (l15 >> 2) + g4 + (l15 & 3);
+    sred[w][o] = gb1;
+    sred[w][kH + o] = gb2;
+    sred[w][2 * kH + o] = gb3;
+    sred[w][3 * kH + o] = gw4;
+    const float l4 = sum16(gb4), ls = sum16(lsum);   // lanes 0..15 hold them
     if (lane == 0) {
         sred[w][4 * kH] = l4;
         sred[w][4 * kH + 1] = ls;
     }
     __syncthreads();
-    for (int i = threadIdx.x; i < 4 * kH + 2; i += kThreads) {
-        float v = sred[0][i] + sred[1][i] + sred[2][i] + sred[3][i];
+    for (int i = threadIdx.x; i < 4 * kH + 2; i += 64 * NW) {
+        float v = 0.0f;
+#pragma unroll
+        for (int k = 0; k < NW; ++k) v += sred[k][i];
         if (i < kH) out[ob1 + i] = v;
         else if (i < 2 * kH) out[ob2 + i - kH] = v;
         else if (i < 3 * kH) out[ob3 + i - 2 * kH] = v;
@@ -437,48 +611,24 @@ __global__ __launch_bounds__(kThreads) void k_mlp_train(const float4* __restrict
     }
 }
 
-// Sums the partial gradients; with adam != 0 applies one Adam step
-// (Kingma & Ba 2015, Algorithm 1) to the FP32 master parameters and refreshes
-// the BF16 copies.  grad_out (optional) receives the summed gradient.  A
-// block owns 64 parameters; its four wavefronts sum interleaved quarters of
-// the partials (four independent accumulators each) and meet in LDS.
-constexpr int kAdamParams = 64;
-__global__ __launch_bounds__(256) void k_mlp_adam(const float* __restrict__ partial, int nparts,
-                                                  const float* __restrict__ loss_partial, float* theta, float* m,
-                                                  float* v, Bf16Weights wb, float lr, float b1, float b2, float eps,
-                                                  float c1, float c2, int adam, float* grad_out,
-                                                  float* loss_out, float inv_batch) {
-    __shared__ float sg[4][kAdamParams];
-    const int pl = threadIdx.x & (kAdamParams - 1), grp = threadIdx.x >> 6;
-    const int p = blockIdx.x * kAdamParams + pl;
-    if (blockIdx.x == 0 && threadIdx.x == 0 && loss_out) {
-        float l = 0.0f;
-        for (int b = 0; b < nparts; ++b) l += loss_partial[b];
-        *loss_out = l * inv_batch;
+// First parameter of the four consecutive ones at value s (a multiple of 4)
+// of a partial gradient vector.
+__device__ __forceinline__ int param_of(int s) {
+    if (s < ob1) {
+        const int l = s / 4 % 64;
+        return oW1 + (16 * (s / 256 % 8) + l % 16) * kH + 16 * (s / 2048) + 4 * (l / 16);
     }
-    float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    if (p < kParams) {
-        int b = grp;
-        for (; b + 12 < nparts; b += 16) {
-#pragma unroll
-            for (int u = 0; u < 4; ++u) acc[u] += partial[(size_t)(b + 4 * u) * kParams + p];
-        }
-        for (; b < nparts; b += 4) acc[0] += partial[(size_t)b * kParams + p];
+    const int o = s >= oW3 && s < ob3 ? oW3 : oW2;
+    if (s >= o && s < o + kH * kH) {
+        const int r = s - o, l = r / 4 % 64;
+        return o + (16 * (r / 256 % 4) + l % 16) * kH + 16 * (r / 1024) + 4 * (l / 16);
     }
-    sg[grp][pl] = (acc[0] + acc[1]) + (acc[2] + acc[3]);
-    __syncthreads();
-    if (grp != 0 || p >= kParams) return;
-    const float g = (sg[0][pl] + sg[1][pl]) + (sg[2][pl] + sg[3][pl]);
-    if (grad_out) grad_out[p] = g;
-    if (!adam) return;
-    float mm = b1 * m[p] + (1.0f - b1) * g;
-    float vv = b2 * v[p] + (1.0f - b2) * g * g;
-    m[p] = mm;
-    v[p] = vv;
-    float mh = mm / c1, vh = vv / c2;
-    float th = theta[p] - lr * mh / (sqrtf(vh) + eps);
-    theta[p] = th;
-    uint16_t hb = f2bf(th);
+    return s;
+}
+
+// BF16 copies of parameter p (value th) in the layouts the products read.
+__device__ __forceinline__ void store_copies(const Bf16Weights& wb, int p, float th) {
+    const uint16_t hb = f2bf(th);
     if (p < ob1) {
         int k = (p - oW1) / kH, nn = (p - oW1) % kH;
         wb.W1T[nn * kK1 + k] = hb;
@@ -494,24 +644,71 @@ __global__ __launch_bounds__(256) void k_mlp_adam(const float* __restrict__ part
     }
 }
 
+// Sums the partial gradients; with adam != 0 applies one Adam step
+// (Kingma & Ba 2015, Algorithm 1) to the FP32 master parameters and refreshes
+// the BF16 copies.  grad_out (optional) receives the summed gradient.  A
+// block owns 64 values of the partial vectors, 16 lanes of four; its 16 lane
+// groups sum every 16th partial each, all loads in flight together, and meet
+// in LDS.  The last block sums the loss.
+constexpr int kAdamParams = 64;
+constexpr int kAdamGroups = 16;
+__global__ __launch_bounds__(256) void k_mlp_adam(const float* __restrict__ partial, int nparts,
+                                                  const float* __restrict__ loss_partial, float* theta, float* m,
+                                                  float* v, Bf16Weights wb, float lr, float b1, float b2, float eps,
+                                                  float c1, float c2, int adam, float* grad_out,
+                                                  float* loss_out, float inv_batch) {
+    __shared__ __align__(16) float4 sg[kAdamGroups][kAdamParams / 4];
+    const int vl = threadIdx.x % (kAdamParams / 4), grp = threadIdx.x / (kAdamParams / 4);
+    if (blockIdx.x == gridDim.x - 1 && loss_out) {
+        // the same order for every launch: thread sums, then the wavefronts'
+        float l = 0.0f;
+        for (int b = threadIdx.x; b < nparts; b += 256) l += loss_partial[b];
+        float* sl = reinterpret_cast<float*>(sg);
+        l = sum16(l);
+        l += __shfl_xor(l, 16, 64);
+        l += __shfl_xor(l, 32, 64);
+        if ((threadIdx.x & 63) == 0) sl[threadIdx.x >> 6] = l;
+        __syncthreads();
+        if (threadIdx.x == 0) *loss_out = ((sl[0] + sl[1]) + (sl[2] + sl[3])) * inv_batch;
+        __syncthreads();
+    }
+    const int s = blockIdx.x * kAdamParams + 4 * vl;
+    float4 acc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if (s < kParams) {
+#pragma unroll 16
+        for (int b = grp; b < nparts; b += kAdamGroups) {
+            const float4 q = *reinterpret_cast<const float4*>(partial + (size_t)b * kPartStride + s);
+            acc.x += q.x;
+            acc.y += q.y;
+            acc.z += q.z;
+            acc.w += q.w;
+        }
+    }
+    sg[grp][vl] = acc;
+    __syncthreads();
+    // one thread per value
+    if (threadIdx.x >= kAdamParams) return;
+    const int p = param_of(blockIdx.x * kAdamParams + (int)(threadIdx.x & ~3u)) + (int)(threadIdx.x & 3u);
+    if (blockIdx.x * kAdamParams + (int)threadIdx.x >= kParams) return;
+    float g = 0.0f;
+#pragma unroll
+    for (int k = 0; k < kAdamGroups; ++k) g += reinterpret_cast<const float*>(sg[k])[threadIdx.x];
+    if (grad_out) grad_out[p] = g;
+    if (!adam) return;
+    float mm = b1 * m[p] + (1.0f - b1) * g;
+    float vv = b2 * v[p] + (1.0f - b2) * g * g;
+    m[p] = mm;
+    v[p] = vv;
+    float mh = mm / c1, vh = vv / c2;
+    float th = theta[p] - lr * mh / (sqrtf(vh) + eps);
+    theta[p] = th;
+    store_copies(wb, p, th);
+}
+
 // BF16 copies of all weights from the FP32 master (after set_params).
 __global__ void k_mlp_copies(const float* theta, Bf16Weights wb) {
     int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= kParams) return;
-    uint16_t hb = f2bf(theta[p]);
-    if (p < ob1) {
-        int k = (p - oW1) / kH, nn = (p - oW1) % kH;
-        wb.W1T[nn * kK1 + k] = hb;
-        wb.W1[k * kH + nn] = hb;
-    } else if (p >= oW2 && p < ob2) {
-        int k = (p - oW2) / kH, nn = (p - oW2) % kH;
-        wb.W2T[nn * kH + k] = hb;
-        wb.W2[k * kH + nn] = hb;
-    } else if (p >= oW3 && p < ob3) {
-        int k = (p - oW3) / kH, nn = (p - oW3) % kH;
-        wb.W3T[nn * kH + k] = hb;
-        wb.W3[k * kH + nn] = hb;
-    }
+    if (p < kParams) store_copies(wb, p, theta[p]);
 }
 
 // Network output y and dy/du of the 64-point tile whose row 16w + lane%16
@@ -1145,14 +1342,14 @@ sph_status sph_mlp_create(const sph_mlp_config* cfg, sph_mlp** out) {
     h->cfg = *cfg;
     int cus = 256;
     (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-    h->nblocks = 2 * cus;
+    h->nblocks = cus;   // one partial gradient vector per CU
     const size_t nb = (size_t)2 * kK1 * kH + (size_t)4 * kH * kH;
     bool ok = hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking) == hipSuccess &&
               hipMalloc(&h->theta, sizeof(float) * kParams) == hipSuccess &&
               hipMalloc(&h->m, sizeof(float) * kParams) == hipSuccess &&
               hipMalloc(&h->v, sizeof(float) * kParams) == hipSuccess &&
               hipMalloc(&h->wbuf, sizeof(uint16_t) * nb) == hipSuccess &&
-              hipMalloc(&h->partial, sizeof(float) * kParams * (size_t)h->nblocks) == hipSuccess &&
+              hipMalloc(&h->partial, sizeof(float) * kPartStride * (size_t)h->nblocks) == hipSuccess &&
               hipMalloc(&h->loss_partial, sizeof(float) * (size_t)h->nblocks) == hipSuccess &&
               hipMalloc(&h->grad, sizeof(float) * kParams) == hipSuccess;
     if (!ok) {
@@ -1239,9 +1436,9 @@ sph_status sph_mlp_set_samples(sph_mlp* h, const float* xyzd, size_t n) {
 
 static sph_status enqueue_pass(sph_mlp* h, uint32_t first, int32_t batch, bool adam, float* grad, float* loss_dev) {
     NetView nv = h->view();
-    const uint32_t tiles = (uint32_t)batch / kTile;
+    const uint32_t tiles = ((uint32_t)batch + kTrainTile - 1) / kTrainTile;
     const int blocks = (int)std::min<uint32_t>(tiles, (uint32_t)h->nblocks);
-    hipLaunchKernelGGL(k_mlp_train, dim3(blocks), dim3(kThreads), 0, h->stream, h->samples, h->nsamples, first,
+    hipLaunchKernelGGL(k_mlp_train, dim3(blocks), dim3(64 * kTrainWaves), 0, h->stream, h->samples, h->nsamples, first,
                        (uint32_t)batch, nv, h->partial, h->loss_partial);
     float c1 = 1.0f, c2 = 1.0f, lr = h->cfg.lr;
     if (adam) {
