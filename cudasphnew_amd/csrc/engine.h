@@ -11,6 +11,7 @@
 
 #include "common.h"
 #include "cell_sort.h"
+#include "host_copy.h"
 #include "kernels.h"
 #include "radix_sort.h"
 
@@ -118,6 +119,10 @@ struct Engine {
     float4* render_pos = nullptr;   // [N] by original id
     float4* render_sub = nullptr;   // [8N] by sub-particle id
     uint8_t* surface = nullptr;     // [N] surface flags by original id, on demand
+    // a field in original-id order on its way to the host, [3 x the largest
+    // scene], allocated on the first read
+    float* read_stage = nullptr;
+    HostCopy reader;
 
     ~Engine();
     void drop_graph();
@@ -136,6 +141,8 @@ struct Engine {
     sph_status fail(sph_status s, const std::string& msg);
     template <class T>
     sph_status alloc(T** p, size_t count);
+    sph_status status_of(uint32_t word);   // error of a device status word
+    sph_status read_floats(int scene, sph_field f, float* dst, size_t nbytes);
     sph_status read_field(int scene, sph_field f, void* dst, size_t bytes_out);
     sph_status upload_params(int scene, const sph_params& p);
     sph_status map_render(sph_render_view* out);

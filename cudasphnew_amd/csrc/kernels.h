@@ -68,6 +68,11 @@ void launch_surface(hipStream_t st, const StepBuffers& b, float cm_thresh, float
 // out[oid[i]] = (pos[i].xyz, vel[i].w) for i < n: positions by original id.
 void launch_export_positions(hipStream_t st, uint32_t n, const float4* pos, const float4* vel, const uint32_t* oid,
                              float4* out);
+// A field of n slots in original-id order: out[3 oid + 0..2] = src.xyz, and
+// out[oid] = vel.w or, for the pressure, stiff (vel.w - rho0).
+void launch_read_xyz(hipStream_t st, uint32_t n, const float4* src, const uint32_t* oid, float* out);
+void launch_read_density(hipStream_t st, uint32_t n, const float4* vel, const uint32_t* oid, bool pressure, float stiff,
+                         float rho0, float* out);
 void launch_force(hipStream_t st, const StepBuffers& b, int lanes, int block = 256);
 // The one-lane and hit-mask variants of a small particle set (team.hip):
 // sixteen lanes per particle, the same results bit for bit.  team_step:

@@ -736,6 +736,31 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(CAP <= 40 ? 5
     }
 }
 
+// A field of one scene in original-id order, as a host read wants it: the
+// device scatters by id (a few us at 256,000 particles), so that the copy to
+// the host is the field alone, straight into the caller's array.  Before, the
+// float4 records and the ids were copied and the host scattered them.
+__global__ __launch_bounds__(kBlock) void k_read_xyz(uint32_t n, const float4* __restrict__ src,
+                                                     const uint32_t* __restrict__ oid, float* __restrict__ out) {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const float4 v = src[i];
+    float* o = out + 3 * (size_t)oid[i];
+    o[0] = v.x;
+    o[1] = v.y;
+    o[2] = v.z;
+}
+
+// Density (channel w), or the pressure stiff (density - rho0).
+__global__ __launch_bounds__(kBlock) void k_read_density(uint32_t n, const float4* __restrict__ vel,
+                                                         const uint32_t* __restrict__ oid, bool pressure, float stiff,
+                                                         float rho0, float* __restrict__ out) {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const float rho = vel[i].w;
+    out[oid[i]] = pressure ? stiff * (rho - rho0) : rho;
+}
+
 // Surface particles (the reference's declared extractSurfaceParticles, on
 // the positions of the last step's force pass): neighbour count including
 // the particle itself and the offset of the neighbourhood's centre of mass,
@@ -894,6 +919,17 @@ void launch_surface(hipStream_t st, const StepBuffers& b, float cm_thresh, float
     if (b.n == 0) return;
     hipLaunchKernelGGL(k_surface, dim3(blocks_for(b.n, kBlock)), dim3(kBlock), 0, st, b.pos_b, b.range, b.n, b.scenes,
                        b.begins, b.nscenes, b.oid_b, cm_thresh, n_thresh, out);
+}
+
+void launch_read_xyz(hipStream_t st, uint32_t n, const float4* src, const uint32_t* oid, float* out) {
+    if (n) hipLaunchKernelGGL(k_read_xyz, dim3(blocks_for(n, kBlock)), dim3(kBlock), 0, st, n, src, oid, out);
+}
+
+void launch_read_density(hipStream_t st, uint32_t n, const float4* vel, const uint32_t* oid, bool pressure, float stiff,
+                         float rho0, float* out) {
+    if (n)
+        hipLaunchKernelGGL(k_read_density, dim3(blocks_for(n, kBlock)), dim3(kBlock), 0, st, n, vel, oid, pressure,
+                           stiff, rho0, out);
 }
 
 void launch_export_positions(hipStream_t st, uint32_t n, const float4* pos, const float4* vel, const uint32_t* oid,

