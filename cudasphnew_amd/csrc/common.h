@@ -149,8 +149,9 @@ __device__ __forceinline__ int range_coord(float x, float dd, float o, float s, 
     float f = ((x + dd) - o) / s;
     if (!(f > 0.0f)) return 0;
     if (f >= 2147483520.0f) return 0;
-    int c = (int)((unsigned)f) % dim;
-    return min(max(c, 0), dim - 1);
+    int c = (int)((unsigned)f);
+    if (c >= dim) c %= dim;   // off the grid: the reference's wrap
+    return c;
 }
 
 __device__ __forceinline__ uint32_t cell_key(const DevScene& S, float x, float y, float z, uint32_t& flags) {

@@ -434,32 +434,69 @@ __device__ __forceinline__ uint32_t near_bits(uint32_t far, int c) {
     return c > 0 ? __builtin_bitreverse32(~far) >> (32 - c) : 0u;
 }
 
-// The candidates [0, cnt) of one row run: adds their poly6 terms to sum and
+// The candidates of a row run, in order, from the wavefront's LDS window or
+// from global memory: (0..2) reads one relative to the current place.
+struct WindowRow {
+    const float* w;
+    __device__ __forceinline__ float3 operator()(int t) const { return make_float3(w[3 * t], w[3 * t + 1], w[3 * t + 2]); }
+    __device__ __forceinline__ void skip4() { w += 12; }
+};
+struct GlobalRow {
+    const F4Buf& pos;
+    uint32_t q;
+    __device__ __forceinline__ float3 operator()(int t) const {
+        const float4 p = pos[q + (uint32_t)t];
+        return make_float3(p.x, p.y, p.z);
+    }
+    __device__ __forceinline__ void skip4() { q += 4u; }
+};
+
+// The next cnt <= 32 candidates of a row run: adds their poly6 terms to sum
+// and returns the "farther than h" bits, newest first.  Groups of four, then
+// the rest under the lane mask: a wavefront's passes are its longest lane's,
+// without a remainder loop whose length is the largest remainder of its lanes.
+template <class Row>
+__device__ __forceinline__ uint32_t density_chunk(Row& at, int cnt, float4 xi, float h2, float& sum) {
+    uint32_t far = 0;
+    auto one = [&](int t) {
+        const float3 p = at(t);
+        density_candidate(p.x, p.y, p.z, xi, h2, sum, far);
+    };
+    int left = cnt;
+#pragma unroll 1
+    for (; left >= 4; left -= 4) {
+        float3 p[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) p[u] = at(u);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) density_candidate(p[u].x, p[u].y, p[u].z, xi, h2, sum, far);
+        at.skip4();
+    }
+    if (left > 0) {
+        one(0);
+        if (left > 1) {
+            one(1);
+            if (left > 2) one(2);
+        }
+    }
+    return far;
+}
+
+// The cnt candidates of one row run: adds their poly6 terms to sum and
 // returns the force-neighbour mask of candidates 0..31 (bit t = candidate t
 // within h; self = the particle's own position in the run, or any value >=
 // cnt).  Each further chunk k of 32 candidates is handed to put(k, mask).
-// at(t) -> (x, y, z) of candidate t.
-template <class At, class Put>
-__device__ __forceinline__ uint32_t density_row(const At& at, int cnt, float4 xi, float h2, uint32_t self, float& sum,
+template <class Row, class Put>
+__device__ __forceinline__ uint32_t density_row(Row at, int cnt, float4 xi, float h2, uint32_t self, float& sum,
                                                 const Put& put) {
-    uint32_t far = 0;
     const int c32 = min(cnt, 32);
-#pragma unroll 4
-    for (int t = 0; t < c32; ++t) {
-        const float3 p = at(t);
-        density_candidate(p.x, p.y, p.z, xi, h2, sum, far);
-    }
-    uint32_t m = near_bits(far, c32);
+    uint32_t m = near_bits(density_chunk(at, c32, xi, h2, sum), c32);
     if (self < (uint32_t)c32) m &= ~(1u << self);
     // rows of a compressed flow
+#pragma unroll 1
     for (int c0 = 32; c0 < cnt; c0 += 32) {
         const int cc = min(cnt - c0, 32);
-        uint32_t f = 0;
-        for (int t = 0; t < cc; ++t) {
-            const float3 p = at(c0 + t);
-            density_candidate(p.x, p.y, p.z, xi, h2, sum, f);
-        }
-        uint32_t mc = near_bits(f, cc);
+        uint32_t mc = near_bits(density_chunk(at, cc, xi, h2, sum), cc);
         const uint32_t sc = self - (uint32_t)c0;
         if (sc < (uint32_t)cc) mc &= ~(1u << sc);
         put((uint32_t)c0 >> 5, mc);
@@ -467,27 +504,109 @@ __device__ __forceinline__ uint32_t density_row(const At& at, int cnt, float4 xi
     return m;
 }
 
-// Window of candidate positions per wavefront, in LDS (x, y, z planes).  The
-// 64 particles of a wavefront are consecutive slots (a few neighbouring cells
-// of one cell row, as a rule), so for each of the nine row offsets their
-// runs lie in one short slot window [lo, hi).  The wavefront copies each
-// window once with coalesced loads, and the candidate loop reads LDS: one
+// LDS written by lanes of a wavefront is read by its other lanes: in program
+// order, no barrier needed beyond keeping the compiler from moving accesses.
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// The nine rows of a particle's neighbour range one after the other, plane by
+// plane: the lane's slot run of row (dk, dj) as row_slots finds it.  What does
+// not depend on the row is formed once (the table indices of the run's cells,
+// at most three as a rule) or once per plane; a row adds a uniform offset to
+// the table's address, its cells are read together, and an empty cell
+// (-1, -1) drops out of the unsigned minimum and the signed maximum by itself.
+struct RowWalk {
+    Rows R;
+    uint32_t c0, c1, c2;   // table indices of row (0, 0)'s first, second, last cell
+    float fj, dz2;         // the row's y cell index, the plane's squared distance
+    bool in_plane;
+
+    __device__ __forceinline__ RowWalk(const DevScene& S, float4 xi) : R(neighbour_rows(S, xi)) {
+        const uint32_t row = S.cell_offset + (uint32_t)(S.nx * (S.ny * R.lz + R.ly));
+        c0 = row + (uint32_t)R.lx;
+        c1 = row + (uint32_t)min(R.lx + 1, R.hx);
+        c2 = row + (uint32_t)R.hx;
+    }
+
+    __device__ __forceinline__ void plane(const DevScene& S, float4 xi, int dk) {
+        const int k = R.lz + dk;
+        const float z0 = S.oz + (float)k * S.cell;
+        const float dz = fmaxf(fmaxf(z0 - xi.z, xi.z - (z0 + S.cell)), 0.0f);
+        dz2 = dz * dz;
+        in_plane = R.hx >= R.lx && k <= R.hz;
+        fj = (float)R.ly;
+    }
+
+    // b = 0xffffffff and e = -1 when the row holds no candidate
+    __device__ __forceinline__ void run(const int2* __restrict__ range, const DevScene& S, float4 xi, int dk, int dj,
+                                        uint32_t& b, int& e) {
+        const float y0 = S.oy + fj * S.cell;
+        const float dy = fmaxf(fmaxf(y0 - xi.y, xi.y - (y0 + S.cell)), 0.0f);
+        const bool in = in_plane && R.ly + dj <= R.hy && !(fmaf(dy, dy, dz2) * 0.99999f > S.h2);
+        fj += 1.0f;
+        b = 0xffffffffu;
+        e = -1;
+        if (!in) return;
+        const int2* __restrict__ row = range + (size_t)(uint32_t)(S.nx * (S.ny * dk + dj));
+        const int2 r0 = row[c0], r1 = row[c1], r2 = row[c2];
+        b = min(min((uint32_t)r0.x, (uint32_t)r1.x), (uint32_t)r2.x);
+        e = max(max(r0.y, r1.y), r2.y);
+        if (c2 - c0 > 2u)   // a support of more than a cell
+            for (uint32_t c = c1 + 1; c < c2; ++c) {
+                const int2 r = row[c];
+                b = min(b, (uint32_t)r.x);
+                e = max(e, r.y);
+            }
+    }
+};
+
+// First and last slot of a wavefront's runs [b, e) of one row (the lanes
+// without a candidate hold b = 0xffffffff, e = -1); false when no lane has
+// one.  The lanes of a wavefront sit in cell order, so as a rule the first
+// lane with a run has the first slot and the last lane the last one; where
+// one has not (a wavefront across two cell rows), the lanes' minimum and
+// maximum are formed.
+__device__ __forceinline__ bool wave_span(uint32_t b, int e, uint32_t& lo, int& hi) {
+    const uint64_t some = __ballot(e >= 0);
+    if (!some) return false;
+    lo = (uint32_t)__builtin_amdgcn_readlane((int)b, __ffsll((unsigned long long)some) - 1);
+    hi = __builtin_amdgcn_readlane(e, 63 - __clzll((long long)some));
+    if (__any(b < lo || e > hi)) {
+        lo = __builtin_amdgcn_readfirstlane(__ockl_wfred_min_u32(b));
+        hi = __builtin_amdgcn_readfirstlane(__ockl_wfred_max_i32(e));
+    }
+    return true;
+}
+
+// Window of candidate positions per wavefront, in LDS (x, y, z consecutive).
+// The 64 particles of a wavefront are consecutive slots (a few neighbouring
+// cells of one cell row, as a rule), so for each of the nine row offsets their
+// runs lie in one short slot window [lo, hi).  The wavefront copies the row's
+// window with coalesced loads and runs the row's candidates from LDS: one
 // global load per particle and row in place of one per particle and
-// candidate, which leaves the pass bound by its arithmetic instead of the
-// texture data path.  A row whose window does not fit in what is left of
-// the wavefront's kWin entries (the first rows fill it; a wavefront that
-// straddles two cell rows or two scenes needs more) reads global memory.
-// kWin trades rows served from LDS against occupancy (the window is the
-// kernel's LDS): measured at 1M particles, 768 entries (all nine rows, four
-// wavefronts per SIMD) 131 us, 640 124 us, 512 121 us, 384 120 us, 256 135 us.
-// Three planes rather than float4 entries: one 12-byte read per candidate
-// without address arithmetic (float4 window) measured 114 us against 109 us
-// at 384 entries (117 us at 320, 122 us at 256) -- the larger window costs
-// more occupancy than the saved instructions gain.
-constexpr int kWin = 384;
+// candidate.  A row whose window is longer than kWin (a wavefront that
+// straddles two cell rows; more than about twice rest density) reads global
+// memory.
+//
+// The pass is bound by its VALU instructions and by the LDS: ten operations
+// and twelve bytes per lane and candidate, and per row some fifty operations
+// that find the run and the window.  Row by row, a window of one row serves
+// all nine (a window filled by the first rows that fit, 384 entries, left four
+// or five of them to global reads), twelve consecutive bytes per candidate
+// need no address arithmetic beyond the loop's, and the loop over rows keeps
+// the code in the instruction cache: 3,756 -> 3,065 VALU instructions per
+// wavefront, 106 -> 86 us at 1M particles near rest density, 101 -> 68 us for
+// 430,000 at twice rest density, 28 -> 22 us for 131,000.  Entries of 16 bytes
+// (one 96-bit read a candidate) take 111 us: the LDS serves them at 15 cycles
+// against 11 for the two reads.  Two or three of the nine rows from global
+// memory instead: 1 to 4% slower steps; windows of 128 or 256: no difference.
+constexpr int kWin = 192;
 
 template <int B, bool ONE>
-__global__ __launch_bounds__(B) void k_density_masks(const float4* __restrict__ pos, float4* __restrict__ vel,
+__global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_density_masks(const float4* __restrict__ pos, float4* __restrict__ vel,
                                                      const int2* __restrict__ range, uint32_t n,
                                                      const DevScene* __restrict__ scenes,
                                                      const uint2* __restrict__ tiles, uint32_t ntiles,
@@ -507,55 +626,49 @@ __global__ __launch_bounds__(B) void k_density_masks(const float4* __restrict__ 
         const DevScene& S = scenes[ws.scene];
         const float4 xi = pos[s];
         const float h2 = S.h2;
-        Rows R = neighbour_rows(S, xi);
-        int rb[9], re[9], wofs[9];
-        bool inlds[9];
-        int fill = 0;
-    #pragma unroll
-        for (int row = 0; row < 9; ++row) {
-            row_slots(range, S, R, row / 3, row % 3, xi, rb[row], re[row]);
-            const bool any = re[row] > rb[row];
-            const int lo = __builtin_amdgcn_readfirstlane(__ockl_wfred_min_i32(any ? rb[row] : 0x7fffffff));
-            const int hi = __builtin_amdgcn_readfirstlane(__ockl_wfred_max_i32(any ? re[row] : -1));
-            inlds[row] = hi > lo && hi - lo <= kWin - fill;
-            wofs[row] = fill - lo;   // LDS index of slot q: q + wofs
-            if (inlds[row]) {
-                for (int i = lane; i < hi - lo; i += 64) {
-                    const float4 p = pos[lo + i];
-                    win[fill + i] = p.x;
-                    win[kWin + fill + i] = p.y;
-                    win[2 * kWin + fill + i] = p.z;
-                }
-                fill += hi - lo;
-            }
-        }
-        // the window is private to the wavefront: its own LDS writes, in
-        // program order, are visible to its later reads
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        RowWalk W(S, xi);
         float sum = 0.0f;
         uint32_t* const cm = chunk_masks(masks, n);
-    #pragma unroll
+        const F4Buf pb(pos);
+    #pragma unroll 1
         for (int row = 0; row < 9; ++row) {
-            const int b = rb[row], cnt = re[row] - rb[row];
+            const int dk = row / 3, dj = row - 3 * dk;   // uniform
+            if (dj == 0) W.plane(S, xi, dk);
+            uint32_t b;
+            int e;
+            W.run(range, S, xi, dk, dj, b, e);
+            uint32_t lo;
+            int hi;
+            const bool some = wave_span(b, e, lo, hi);
+            const int cnt = max(e - (int)b, 0);   // 0 for an empty row: e = -1, b = -1
+            b = cnt > 0 ? b : 0u;
             // the particle's own slot is not a force neighbour
-            const uint32_t self = s - (uint32_t)b;
+            const uint32_t self = s - b;
             const bool keep = live && cnt <= kRowMaxCands;
             auto put = [&](uint32_t k, uint32_t mk) {
                 if (keep) cm[chunk_at(n, k, row, s)] = mk;
             };
-            uint32_t m;
-            if (inlds[row]) {
-                const float* w = win + (b + wofs[row]);
-                m = density_row([&](int t) { return make_float3(w[t], w[kWin + t], w[2 * kWin + t]); }, cnt, xi, h2,
-                                self, sum, put);
-            } else {
-                const F4Buf pb(pos);
-                m = density_row([&](int t) { const float4 p = pb[b + t]; return make_float3(p.x, p.y, p.z); }, cnt,
-                                xi, h2, self, sum, put);
+            uint32_t m = 0;
+            if (some && hi - (int)lo <= kWin) {
+                const int span = hi - (int)lo;
+                float* mine = win + 3 * lane;
+                const uint32_t q = lo + (uint32_t)lane;
+    #pragma unroll
+                for (int i = 0; i < kWin / 64; ++i)
+                    if (lane < span - 64 * i) {
+                        const float4 p = pb[q + 64u * i];
+                        mine[192 * i] = p.x;
+                        mine[192 * i + 1] = p.y;
+                        mine[192 * i + 2] = p.z;
+                    }
+                wave_sync();
+                // a lane without a run reads nothing; its place is any
+                m = density_row(WindowRow{win + __umul24(b - lo, 3)}, cnt, xi, h2, self, sum, put);
+                wave_sync();   // the next row's window replaces this one
+            } else if (some) {
+                m = density_row(GlobalRow{pb, b}, cnt, xi, h2, self, sum, put);
             }
-            const uint64_t w = (uint64_t)(uint32_t)b << 32 | m;
+            const uint64_t w = (uint64_t)b << 32 | m;
             if (live)
                 masks[(size_t)row * n + s] =
                     cnt <= 32 ? w : (keep ? w | (uint64_t)((cnt - 1) >> 5) << 60 : kRowLong);

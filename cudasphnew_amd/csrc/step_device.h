@@ -70,7 +70,7 @@ __device__ __forceinline__ void row_slots(const int2* __restrict__ range, const 
     const float y0 = S.oy + (float)j * S.cell, z0 = S.oz + (float)k * S.cell;
     const float dy = fmaxf(fmaxf(y0 - xi.y, xi.y - (y0 + S.cell)), 0.0f);
     const float dz = fmaxf(fmaxf(z0 - xi.z, xi.z - (z0 + S.cell)), 0.0f);
-    if ((dy * dy + dz * dz) * 0.99999f > S.h2) return;
+    if (fmaf(dy, dy, dz * dz) * 0.99999f > S.h2) return;
     uint32_t rowbase = S.cell_offset + (uint32_t)(S.nx * (S.ny * k + j));
     row_run(range, rowbase, R.lx, R.hx, b, e);
     if (e < b) { b = 0; e = 0; }
