@@ -47,6 +47,7 @@ SOURCES = [
     ("scene.cpp", "host"),
     ("radix_sort.hip", "device"),
     ("cell_sort.hip", "device"),
+    ("small_sort.hip", "device"),
     ("kernels.hip", "device"),
     ("team.hip", "device"),
     ("twoscale.hip", "device"),

@@ -41,6 +41,10 @@ struct StepBuffers {
     // density pass and read by the force pass; null = neighbour loops
     // without masks
     uint64_t* masks = nullptr;
+    // the force pass's positions and velocities go to pos_a[id], vel_a[id]
+    // instead of storage order (one-lane variant; the last step of a call that
+    // returns its particles by id)
+    bool by_id = false;
     // two-scale split flags, set by the hit-mask density pass (state == null: none)
     SplitRefs split = {nullptr, nullptr, nullptr, nullptr};
     // learned boundary records (mode == null: grid everywhere)
@@ -74,6 +78,19 @@ void launch_read_xyz(hipStream_t st, uint32_t n, const float4* src, const uint32
 void launch_read_density(hipStream_t st, uint32_t n, const float4* vel, const uint32_t* oid, bool pressure, float stiff,
                          float rho0, float* out);
 void launch_force(hipStream_t st, const StepBuffers& b, int lanes, int block = 256);
+// Cell sort and reorder of a small particle set in one workgroup
+// (small_sort.hip): whether a set takes it, and the launches -- sorted keys,
+// ranges of all cells, sorted copies.  f.scene != null: the first step of a
+// call without a handle; the keys are formed from pos_a with S, the ids are the
+// indices, and the scene record, slot range and status word are written.
+struct SmallFirst {
+    DevScene* scene = nullptr;
+    uint32_t* begins = nullptr;
+    uint32_t* status = nullptr;
+};
+bool small_sort(uint32_t n, uint64_t cells);
+void launch_small_sort(hipStream_t st, const StepBuffers& b, uint32_t cells, const DevScene& S,
+                       const SmallFirst& f = SmallFirst());
 // The one-lane and hit-mask variants of a small particle set (team.hip):
 // sixteen lanes per particle, the same results bit for bit.  team_step:
 // whether this step's buffers take them, the same answer for both passes.

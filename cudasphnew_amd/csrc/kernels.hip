@@ -257,7 +257,7 @@ __global__ __launch_bounds__(B) void k_force(
     const float4* __restrict__ grid4, const float* __restrict__ gridd, const uint32_t* __restrict__ oid_b,
     const uint8_t* __restrict__ state_b, float4* __restrict__ acc, float4* __restrict__ pos_out,
     float4* __restrict__ vel_out, uint32_t* __restrict__ oid_out, uint8_t* __restrict__ state_out,
-    uint32_t* __restrict__ key_out, uint32_t* __restrict__ status, NeuralRefs nr) {
+    uint32_t* __restrict__ key_out, uint32_t* __restrict__ status, NeuralRefs nr, bool by_id) {
     uint32_t s = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
     if (s >= n) return;
     const DevScene& S = scene_for<ONE>(scenes, begins, nscenes, s);
@@ -292,7 +292,7 @@ __global__ __launch_bounds__(B) void k_force(
             }
         }
     force_finish(S, s, xi, vi, a, grid4, gridd, oid_b, state_b, acc, pos_out, vel_out, oid_out, state_out, key_out,
-                 status, nr);
+                 status, nr, by_id);
 }
 
 // Wavefront-cooperative force.  Per round, L adjacent lanes share a particle:
@@ -1079,11 +1079,11 @@ void launch_force(hipStream_t st, const StepBuffers& b, int lanes, int block) {
     case 16: hipLaunchKernelGGL(k_force_coop<16>, g, t, 0, st, SPH_FORCE_ARGS); break;
     default:
         if (small) {
-            if (one) hipLaunchKernelGGL((k_force<128, true>), dim3(blocks_for(b.n, 128)), dim3(128), 0, st, SPH_FORCE_ARGS);
-            else hipLaunchKernelGGL((k_force<128, false>), dim3(blocks_for(b.n, 128)), dim3(128), 0, st, SPH_FORCE_ARGS);
+            if (one) hipLaunchKernelGGL((k_force<128, true>), dim3(blocks_for(b.n, 128)), dim3(128), 0, st, SPH_FORCE_ARGS, b.by_id);
+            else hipLaunchKernelGGL((k_force<128, false>), dim3(blocks_for(b.n, 128)), dim3(128), 0, st, SPH_FORCE_ARGS, b.by_id);
         } else {
-            if (one) hipLaunchKernelGGL((k_force<kBlock, true>), g, t, 0, st, SPH_FORCE_ARGS);
-            else hipLaunchKernelGGL((k_force<kBlock, false>), g, t, 0, st, SPH_FORCE_ARGS);
+            if (one) hipLaunchKernelGGL((k_force<kBlock, true>), g, t, 0, st, SPH_FORCE_ARGS, b.by_id);
+            else hipLaunchKernelGGL((k_force<kBlock, false>), g, t, 0, st, SPH_FORCE_ARGS, b.by_id);
         }
         break;
     }

@@ -387,7 +387,11 @@ void Engine::enqueue_step(bool two_scale) {
     // the counting sort clears the previous step's cells itself
     if (cells_valid && !use_cell_sort) launch_cells_clear(stream, b);
     mark(kStageClear);
-    if (use_cell_sort) {
+    if (use_cell_sort && small_sort(N, total_cells)) {
+        // sort, cell ranges and reorder of a small set in one workgroup
+        launch_small_sort(stream, b, total_cells, hscenes[0]);
+        mark(kStageSort);
+    } else if (use_cell_sort) {
         // the counting sort writes the cell ranges itself
         csort.sort(stream, key, N, skey, perm, range, cells_valid);
         mark(kStageSort);
@@ -397,7 +401,7 @@ void Engine::enqueue_step(bool two_scale) {
         launch_cells(stream, b);
         mark(kStageCells);
     }
-    launch_reorder(stream, b);
+    if (!use_cell_sort || !small_sort(N, total_cells)) launch_reorder(stream, b);
     mark(kStageReorder);
     // a two-scale step's split flags come from the hit-mask density pass
     if (two_scale && b.masks) b.split = twoscale_split_refs(*this);

@@ -139,7 +139,7 @@ __device__ __forceinline__ void force_finish(const DevScene& S, uint32_t s, floa
                                              float4* __restrict__ acc, float4* __restrict__ pos_out,
                                              float4* __restrict__ vel_out, uint32_t* __restrict__ oid_out,
                                              uint8_t* __restrict__ state_out, uint32_t* __restrict__ key_out,
-                                             uint32_t* __restrict__ status, const NeuralRefs& nr) {
+                                             uint32_t* __restrict__ status, const NeuralRefs& nr, bool by_id = false) {
     const float rhoi = vi.w;
     const float cpf = -S.mass * S.grad_spiky, cvf = S.mu * S.mass * S.lapl_visc;
     float Fx = fmaf(cvf, a.fvx, cpf * a.fpx), Fy = fmaf(cvf, a.fvy, cpf * a.fpy), Fz = fmaf(cvf, a.fvz, cpf * a.fpz);
@@ -222,10 +222,11 @@ __device__ __forceinline__ void force_finish(const DevScene& S, uint32_t s, floa
     if (!(isfinite(px) && isfinite(py) && isfinite(pz) && isfinite(vx) && isfinite(vy) && isfinite(vz)))
         flags |= kStatusNonFinite;
     if (flags) atomicOr(status, flags);
-    pos_out[s] = make_float4(px, py, pz, rhoi);
-    vel_out[s] = make_float4(vx, vy, vz, rhoi);
+    const uint32_t id = oid_b[s], at = by_id ? id : s;
+    pos_out[at] = make_float4(px, py, pz, rhoi);
+    vel_out[at] = make_float4(vx, vy, vz, rhoi);
     key_out[s] = kk;
-    oid_out[s] = oid_b[s];
+    oid_out[s] = id;
     if (state_out) state_out[s] = state_b[s];
 }
 

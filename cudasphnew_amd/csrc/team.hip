@@ -226,7 +226,7 @@ __global__ __launch_bounds__(kBlock) void k_force_team(
     const float4* __restrict__ grid4, const float* __restrict__ gridd, const uint32_t* __restrict__ oid_b,
     const uint8_t* __restrict__ state_b, float4* __restrict__ acc, float4* __restrict__ pos_out,
     float4* __restrict__ vel_out, uint32_t* __restrict__ oid_out, uint8_t* __restrict__ state_out,
-    uint32_t* __restrict__ key_out, uint32_t* __restrict__ status, NeuralRefs nr) {
+    uint32_t* __restrict__ key_out, uint32_t* __restrict__ status, NeuralRefs nr, bool by_id) {
     __shared__ int s_list[kTeams][kList];
     __shared__ __align__(16) float s_terms[kBlock / 64][11 * kTermStride];
     __shared__ float s_sum[10][kTeams];
@@ -299,7 +299,7 @@ __global__ __launch_bounds__(kBlock) void k_force_team(
 #pragma unroll
     for (int t = 0; t < 10; ++t) av[t] = s_sum[t][threadIdx.x];
     force_finish(S, p, pos[p], vel[p], a, grid4, gridd, oid_b, state_b, acc, pos_out, vel_out, oid_out, state_out,
-                 key_out, status, nr);
+                 key_out, status, nr, by_id);
 }
 
 unsigned team_blocks(uint32_t n) { return (n + kTeams - 1) / kTeams; }
@@ -314,7 +314,7 @@ template <bool MASKS, bool ONE>
 void force_team(hipStream_t st, const StepBuffers& b) {
     hipLaunchKernelGGL((k_force_team<MASKS, ONE>), dim3(team_blocks(b.n)), dim3(kBlock), 0, st, b.pos_b, b.vel_b,
                        b.range, b.n, b.scenes, b.begins, b.nscenes, b.grid4, b.gridd, b.oid_b, b.state_b, b.acc,
-                       b.pos_a, b.vel_a, b.oid_a, b.state_a, b.key, b.status, b.nr);
+                       b.pos_a, b.vel_a, b.oid_a, b.state_a, b.key, b.status, b.nr, b.by_id);
 }
 
 // Teams issue about four times the instructions of one thread per particle,
