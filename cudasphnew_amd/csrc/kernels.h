@@ -41,9 +41,11 @@ struct StepBuffers {
     // density pass and read by the force pass; null = neighbour loops
     // without masks
     uint64_t* masks = nullptr;
+    // masks with the one-lane variants' results bit for bit (one scene)
+    bool plain_masks = false;
     // the force pass's positions and velocities go to pos_a[id], vel_a[id]
-    // instead of storage order (one-lane variant; the last step of a call that
-    // returns its particles by id)
+    // instead of storage order (the one-lane, team and masks variants; the last
+    // step of a call that returns its particles by id)
     bool by_id = false;
     // two-scale split flags, set by the hit-mask density pass (state == null: none)
     SplitRefs split = {nullptr, nullptr, nullptr, nullptr};

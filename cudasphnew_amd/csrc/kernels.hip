@@ -455,12 +455,12 @@ struct GlobalRow {
 // and returns the "farther than h" bits, newest first.  Groups of four, then
 // the rest under the lane mask: a wavefront's passes are its longest lane's,
 // without a remainder loop whose length is the largest remainder of its lanes.
-template <class Row>
+template <bool GAP, class Row>
 __device__ __forceinline__ uint32_t density_chunk(Row& at, int cnt, float4 xi, float h2, float& sum) {
     uint32_t far = 0;
     auto one = [&](int t) {
         const float3 p = at(t);
-        density_candidate(p.x, p.y, p.z, xi, h2, sum, far);
+        density_candidate<GAP>(p.x, p.y, p.z, xi, h2, sum, far);
     };
     int left = cnt;
 #pragma unroll 1
@@ -469,7 +469,7 @@ __device__ __forceinline__ uint32_t density_chunk(Row& at, int cnt, float4 xi, f
 #pragma unroll
         for (int u = 0; u < 4; ++u) p[u] = at(u);
 #pragma unroll
-        for (int u = 0; u < 4; ++u) density_candidate(p[u].x, p[u].y, p[u].z, xi, h2, sum, far);
+        for (int u = 0; u < 4; ++u) density_candidate<GAP>(p[u].x, p[u].y, p[u].z, xi, h2, sum, far);
         at.skip4();
     }
     if (left > 0) {
@@ -486,17 +486,17 @@ __device__ __forceinline__ uint32_t density_chunk(Row& at, int cnt, float4 xi, f
 // returns the force-neighbour mask of candidates 0..31 (bit t = candidate t
 // within h; self = the particle's own position in the run, or any value >=
 // cnt).  Each further chunk k of 32 candidates is handed to put(k, mask).
-template <class Row, class Put>
+template <bool GAP, class Row, class Put>
 __device__ __forceinline__ uint32_t density_row(Row at, int cnt, float4 xi, float h2, uint32_t self, float& sum,
                                                 const Put& put) {
     const int c32 = min(cnt, 32);
-    uint32_t m = near_bits(density_chunk(at, c32, xi, h2, sum), c32);
+    uint32_t m = near_bits(density_chunk<GAP>(at, c32, xi, h2, sum), c32);
     if (self < (uint32_t)c32) m &= ~(1u << self);
     // rows of a compressed flow
 #pragma unroll 1
     for (int c0 = 32; c0 < cnt; c0 += 32) {
         const int cc = min(cnt - c0, 32);
-        uint32_t mc = near_bits(density_chunk(at, cc, xi, h2, sum), cc);
+        uint32_t mc = near_bits(density_chunk<GAP>(at, cc, xi, h2, sum), cc);
         const uint32_t sc = self - (uint32_t)c0;
         if (sc < (uint32_t)cc) mc &= ~(1u << sc);
         put((uint32_t)c0 >> 5, mc);
@@ -605,7 +605,9 @@ __device__ __forceinline__ bool wave_span(uint32_t b, int e, uint32_t& lo, int& 
 // memory instead: 1 to 4% slower steps; windows of 128 or 256: no difference.
 constexpr int kWin = 192;
 
-template <int B, bool ONE>
+// PLAIN: the arithmetic of k_density, bit for bit (the pair of masks kernels
+// in place of the one-lane kernels).
+template <int B, bool ONE, bool PLAIN = false>
 __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_density_masks(const float4* __restrict__ pos, float4* __restrict__ vel,
                                                      const int2* __restrict__ range, uint32_t n,
                                                      const DevScene* __restrict__ scenes,
@@ -663,10 +665,10 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(8, 8))) void 
                     }
                 wave_sync();
                 // a lane without a run reads nothing; its place is any
-                m = density_row(WindowRow{win + __umul24(b - lo, 3)}, cnt, xi, h2, self, sum, put);
+                m = density_row<PLAIN>(WindowRow{win + __umul24(b - lo, 3)}, cnt, xi, h2, self, sum, put);
                 wave_sync();   // the next row's window replaces this one
             } else if (some) {
-                m = density_row(GlobalRow{pb, b}, cnt, xi, h2, self, sum, put);
+                m = density_row<PLAIN>(GlobalRow{pb, b}, cnt, xi, h2, self, sum, put);
             }
             const uint64_t w = (uint64_t)b << 32 | m;
             if (live)
@@ -725,7 +727,10 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(8, 8))) void 
 // CAP 40 (5 wavefronts, 85 VGPRs) 127 us, 48 (4) 132 us, 32 at 6 wavefronts
 // spills and takes 139 us (156 us with two gathers in flight instead of
 // three).
-template <int CAP, int B, bool ONE>
+//
+// PLAIN: the sums of k_force, bit for bit: a particle with a row past
+// kRowMaxCands scans all its rows in order.
+template <int CAP, int B, bool ONE, bool PLAIN = false>
 __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(CAP <= 40 ? 5 : (CAP <= 48 ? 4 : 3), 8))) void k_force_masks(
     const float4* __restrict__ pos, const float4* __restrict__ vel, const int2* __restrict__ range, uint32_t n,
     const DevScene* __restrict__ scenes, const uint2* __restrict__ tiles, uint32_t ntiles,
@@ -733,7 +738,7 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(CAP <= 40 ? 5
     const uint8_t* __restrict__ state_b, float4* __restrict__ acc, float4* __restrict__ pos_out,
     float4* __restrict__ vel_out, uint32_t* __restrict__ oid_out, uint8_t* __restrict__ state_out,
     uint32_t* __restrict__ key_out, uint32_t* __restrict__ status, const uint64_t* __restrict__ masks,
-    NeuralRefs nr) {
+    NeuralRefs nr, bool by_id) {
     // one column per thread: no barrier needed, consecutive threads hit
     // consecutive banks
     __shared__ uint16_t s_list[CAP][B];
@@ -760,6 +765,12 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(CAP <= 40 ? 5
                 last |= lr ? 0u : row_last_chunk(mk[row]) << (2 * row);
                 s_base[row][tid] = (int)row_first(mk[row]);
             }
+        }
+        if (PLAIN && long_rows) {
+            long_rows = 0x1FFu;
+            last = 0u;
+#pragma unroll
+            for (int row = 0; row < 9; ++row) bits[row] = 0u;
         }
         const uint32_t* const cm = chunk_masks(masks, n);
         const float4 xi = pos[s];
@@ -813,19 +824,19 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(CAP <= 40 ? 5
                 float4 x2 = pb[q], v2 = vb[q];
                 int k = 0;
                 for (; k + 3 < m; k += 3) {
-                    pair_terms<true>(a, xi, vi, rhoi, Ai, h, h2, S.stiff, kr0, x0, v0);
+                    pair_terms<!PLAIN>(a, xi, vi, rhoi, Ai, h, h2, S.stiff, kr0, x0, v0);
                     q = slot(k + 3);
                     x0 = pb[q]; v0 = vb[q];
-                    pair_terms<true>(a, xi, vi, rhoi, Ai, h, h2, S.stiff, kr0, x1, v1);
+                    pair_terms<!PLAIN>(a, xi, vi, rhoi, Ai, h, h2, S.stiff, kr0, x1, v1);
                     q = slot(k + 4);
                     x1 = pb[q]; v1 = vb[q];
-                    pair_terms<true>(a, xi, vi, rhoi, Ai, h, h2, S.stiff, kr0, x2, v2);
+                    pair_terms<!PLAIN>(a, xi, vi, rhoi, Ai, h, h2, S.stiff, kr0, x2, v2);
                     q = slot(k + 5);
                     x2 = pb[q]; v2 = vb[q];
                 }
-                pair_terms<true>(a, xi, vi, rhoi, Ai, h, h2, S.stiff, kr0, x0, v0);
-                if (k + 1 < m) pair_terms<true>(a, xi, vi, rhoi, Ai, h, h2, S.stiff, kr0, x1, v1);
-                if (k + 2 < m) pair_terms<true>(a, xi, vi, rhoi, Ai, h, h2, S.stiff, kr0, x2, v2);
+                pair_terms<!PLAIN>(a, xi, vi, rhoi, Ai, h, h2, S.stiff, kr0, x0, v0);
+                if (k + 1 < m) pair_terms<!PLAIN>(a, xi, vi, rhoi, Ai, h, h2, S.stiff, kr0, x1, v1);
+                if (k + 2 < m) pair_terms<!PLAIN>(a, xi, vi, rhoi, Ai, h, h2, S.stiff, kr0, x2, v2);
             }
         } while (m == CAP);   // a full list: hits may remain
         if (long_rows) {
@@ -845,7 +856,7 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(CAP <= 40 ? 5
             }
         }
         force_finish(S, s, xi, vi, a, grid4, gridd, oid_b, state_b, acc, pos_out, vel_out, oid_out, state_out, key_out,
-                     status, nr);
+                     status, nr, by_id);
     }
 }
 
@@ -1001,6 +1012,12 @@ static void launch_density_one_lane(hipStream_t st, const StepBuffers& b) {
 void launch_density(hipStream_t st, const StepBuffers& b, int lanes, int block) {
     const bool small = block == 128, one = b.nscenes == 1;
     if ((b.masks || lanes == 1) && team_step(b)) return launch_density_team(st, b);
+    if (b.masks && b.plain_masks) {
+        hipLaunchKernelGGL((k_density_masks<kBlock, true, true>), dim3(mask_blocks<kBlock, true>(b)), dim3(kBlock), 0,
+                           st, b.pos_b, b.vel_b, b.range, b.n, b.scenes, b.tiles, b.ntiles, b.grid4, b.masks, b.nr,
+                           b.split);
+        return;
+    }
     if (b.masks) {
         if (small) one ? launch_density_masks<128, true>(st, b) : launch_density_masks<128, false>(st, b);
         else one ? launch_density_masks<kBlock, true>(st, b) : launch_density_masks<kBlock, false>(st, b);
@@ -1026,7 +1043,7 @@ void launch_density(hipStream_t st, const StepBuffers& b, int lanes, int block) 
 
 #define SPH_FORCE_ARGS_M                                                                                            \
     b.pos_b, b.vel_b, b.range, b.n, b.scenes, b.tiles, b.ntiles, b.grid4, b.gridd, b.oid_b, b.state_b, b.acc,      \
-        b.pos_a, b.vel_a, b.oid_a, b.state_a, b.key, b.status, b.masks, b.nr
+        b.pos_a, b.vel_a, b.oid_a, b.state_a, b.key, b.status, b.masks, b.nr, b.by_id
 
 void launch_surface(hipStream_t st, const StepBuffers& b, float cm_thresh, float n_thresh, uint8_t* out) {
     if (b.n == 0) return;
@@ -1065,6 +1082,11 @@ static void launch_force_masks(hipStream_t st, const StepBuffers& b, int cap) {
 void launch_force(hipStream_t st, const StepBuffers& b, int lanes, int block) {
     const bool small = block == 128, one = b.nscenes == 1;
     if ((b.masks || lanes == 1) && team_step(b)) return launch_force_team(st, b);
+    if (b.masks && b.plain_masks) {
+        hipLaunchKernelGGL((k_force_masks<48, kBlock, true, true>), dim3(mask_blocks<kBlock, true>(b)), dim3(kBlock),
+                           0, st, SPH_FORCE_ARGS_M);
+        return;
+    }
     if (b.masks) {
         // lanes selects the LDS hit-list capacity of the hit-mask variant
         if (small) one ? launch_force_masks<128, true>(st, b, lanes) : launch_force_masks<128, false>(st, b, lanes);

@@ -260,12 +260,22 @@ __device__ __forceinline__ float density_gap(float4 xi, float4 xj, float h2) {
 // an exact result, which keeps its sign (and an exact zero is +0), so d's
 // sign bit is set exactly when this d is negative, i.e. when the candidate's
 // poly6 term is zero: the bit is that "farther than h" bit and one funnel
-// shift per candidate builds the mask.
+// shift per candidate builds the mask.  GAP: the d of density_gap instead, and
+// the bit is exactly !(0 < r^2 <= h^2), the test of the loops without masks,
+// whatever the values (three instructions more).
+template <bool GAP = false>
 __device__ __forceinline__ void density_candidate(float xjx, float xjy, float xjz, float4 xi, float h2, float& sum,
                                                   uint32_t& far) {
     float dx = xjx - xi.x, dy = xjy - xi.y, dz = xjz - xi.z;
-    float d = fmaf(-dx, dx, fmaf(-dy, dy, fmaf(-dz, dz, h2)));
-    far = __builtin_amdgcn_alignbit(far, __float_as_uint(d), 31);
+    float d, bit;
+    if (GAP) {
+        const float r2 = sq3(dx, dy, dz);
+        d = h2 - r2;
+        bit = r2 > 0.0f ? d : -1.0f;
+    } else {
+        bit = d = fmaf(-dx, dx, fmaf(-dy, dy, fmaf(-dz, dz, h2)));
+    }
+    far = __builtin_amdgcn_alignbit(far, __float_as_uint(bit), 31);
     d = fmaxf(d, 0.0f);
     sum += d * d * d;
 }

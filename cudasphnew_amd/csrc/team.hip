@@ -322,9 +322,11 @@ void force_team(hipStream_t st, const StepBuffers& b) {
 // the dam break's block, both passes and the sort, us a step, teams against
 // one thread: 35 / 78 at 4,000 particles, 46 / 78 at 16,384, 64 / 79 at
 // 32,768, 85 / 77 at 50,000 (twice rest density: 132 / 141 there); against
-// the hit-mask pair 55 / 63 at 16,384, 72 / 64 at 32,768.  A two-scale step
-// needs the hit-mask density pass's row words and split flags.
-constexpr uint32_t kTeamMax = 40960, kTeamMaxMasks = 24576;
+// the hit-mask pair, two steps and a read of the positions, 118 / 125 at
+// 16,384, 132 / 125 at 20,000 (twice rest density 150 / 187 at 16,384, 204 /
+// 188 at 24,000).  A two-scale step needs the hit-mask density pass's row
+// words and split flags.
+constexpr uint32_t kTeamMax = 40960, kTeamMaxMasks = 18432;
 
 }  // namespace
 

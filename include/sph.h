@@ -749,9 +749,9 @@ sph_status sph_boundary_map_load(const char* path, sph_boundary_map_config* cfg,
  * device memory.  The call allocates nothing, copies nothing between host
  * and device and does not synchronise: kernels only, on `stream` (a
  * hipStream_t; NULL = the null stream).  Every other buffer (keys, orders,
- * sorted copies, cell table, sort counts: SPH_NOALLOC_SCRATCH_BYTES) lives in
- * one static device array of the library, one per GPU, held until the
- * process ends.  All calls on one GPU share it: each call clears what must
+ * sorted copies, cell table, sort counts, neighbour masks:
+ * SPH_NOALLOC_SCRATCH_BYTES) lives in one static device array of the
+ * library, one per GPU, held until the process ends.  All calls on one GPU share it: each call clears what must
  * start cleared, but calls that overlap on one GPU (two streams, two host
  * threads) race and give undefined results.  The first call on a device
  * looks the array's address up (not a stream operation): make it outside
@@ -771,7 +771,7 @@ sph_status sph_boundary_map_load(const char* path, sph_boundary_map_config* cfg,
  * original id, bit for bit. */
 #define SPH_NOALLOC_MAX_PARTICLES 262144u
 #define SPH_NOALLOC_MAX_CELLS 1048576u
-#define SPH_NOALLOC_SCRATCH_BYTES 39848960u
+#define SPH_NOALLOC_SCRATCH_BYTES 87034880u
 typedef struct sph_device_boundary {
     float origin[3];
     float spacing;
