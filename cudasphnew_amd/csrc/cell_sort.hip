@@ -2,23 +2,26 @@
 //
 //   k_cs_count    one atomic per run of equal keys in a wavefront: the
 //                 cells' counts and each particle's arrival rank in its cell;
-//                 flags the 4096-cell blocks that hold a key
-//   k_cs_reduce   totals of 4096-cell blocks (16 counts per thread, read as
-//                 four 16-byte vectors); an unflagged block is empty and
-//                 reads nothing (a fluid filling a tenth of the domain's
-//                 cells touches about a tenth of the blocks)
+//                 and the totals of 4096-cell blocks, added up in LDS per
+//                 workgroup of 1,024 first and then in one of eight copies
+//                 (workgroups of 256 and a single copy serialise: 8.2 us in
+//                 place of 4.9 at 250,000 particles, 9.4 and 6.9 at 1M)
 //   k_cs_ranges   cell starts = offset of the block (sum of the totals of
 //                 the blocks before it, read by the whole workgroup) + scan
-//                 inside the block; writes range[k] of every occupied cell
-//                 and clears its count and the block's flag
-//   k_cs_scatter  slot = start of the cell + arrival rank
-// (Block totals accumulated by atomics in k_cs_count were measured slower:
-// neighbouring wavefronts add to the same total and serialise.)
-// Two streaming reads of the count array (4 bytes per cell) replace the
+//                 inside the block (16 counts per thread, read as four 16-byte
+//                 vectors); writes range[k] of every occupied cell and clears
+//                 its count; a block with total 0 reads nothing (a fluid
+//                 filling a tenth of the domain's cells touches about a tenth
+//                 of the blocks)
+//   k_cs_scatter  slot = start of the cell + arrival rank; clears the totals
+// One streaming read of the count array (4 bytes per cell) replaces the
 // three count / scan / scatter passes of an LSD radix sort over the keys and
-// the separate cell-range pass.  The arrival order inside a cell is not
-// deterministic; the reorder pass ranks each cell by original id, so the
-// sorted state is.
+// the separate cell-range pass.  The passes are short (2.5 to 3 us each, most
+// of it the launch, up to 260,000 particles), so their number counts: without
+// a pass of its own for the totals four steps of 250,000 particles take 316
+// in place of 326 us, two of 16,384 121 in place of 124.  The arrival order
+// inside a cell is not deterministic; the reorder pass ranks each cell by
+// original id, so the sorted state is.
 #include "cell_sort.h"
 
 namespace sph {
@@ -28,18 +31,25 @@ namespace {
 constexpr int kCsThreads = 256;
 constexpr int kCsPerThread = 16;
 constexpr int kCsBlockCells = kCsThreads * kCsPerThread;   // 4096
+constexpr int kCountThreads = 1024;                        // k_cs_count
+constexpr uint32_t kCopies = kCsCopies;                    // of each block's total
 
 // The keys arrive nearly sorted (the storage order is the last step's cell
 // order), so a wavefront holds a few runs of equal keys: the first lane of
 // each run adds the run's length with one atomic and hands the old count to
 // the run, whose lanes rank themselves by their offset in it.  Equal keys
 // in separate runs take separate atomics, which is still exact.
-__global__ __launch_bounds__(kCsThreads) void k_cs_count(const uint32_t* __restrict__ keys, uint32_t n_host,
-                                                         const uint32_t* __restrict__ n_dev,
+// FIRST: the keys are formed here, from the positions.
+template <bool FIRST>
+__global__ __launch_bounds__(kCountThreads) void k_cs_count(KeysFirst first, uint32_t* __restrict__ keys,
+                                                         uint32_t n_host, const uint32_t* __restrict__ n_dev,
                                                          uint32_t* __restrict__ cnt, uint32_t* __restrict__ rank,
-                                                         uint32_t* __restrict__ used,
+                                                         uint32_t* __restrict__ bsum, uint32_t blocks,
                                                          const uint32_t* __restrict__ prev_skey, uint32_t prev_n,
                                                          int2* __restrict__ range) {
+    // totals of the kCsThreads blocks from `first_block` on
+    __shared__ uint32_t s_tot[kCsThreads];
+    __shared__ uint32_t s_first;
     const uint32_t n = n_dev ? *n_dev : n_host;
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     // invalidate the cells of the previous sort (its sorted keys, prev_n of
@@ -48,27 +58,53 @@ __global__ __launch_bounds__(kCsThreads) void k_cs_count(const uint32_t* __restr
         const uint32_t pk = prev_skey[i];
         if (i == 0 || prev_skey[i - 1] != pk) range[pk] = make_int2(-1, -1);
     }
-    if ((i & ~63u) >= n) return;   // the whole wavefront lies past the end
+    if (blockIdx.x * blockDim.x >= n) return;   // the whole workgroup lies past the end
     const int lane = threadIdx.x & 63;
     const bool valid = i < n;
-    const uint32_t k = valid ? keys[i] : 0xFFFFFFFFu;
+    uint32_t k = 0xFFFFFFFFu;
+    if (valid) {
+        if (FIRST) {
+            const float4 p = first.pos[i];
+            uint32_t flags = 0;
+            keys[i] = k = cell_key(first.scene, p.x, p.y, p.z, flags);
+            if (flags) atomicOr(first.status, flags);
+        } else {
+            k = keys[i];
+        }
+    }
+    if (threadIdx.x < kCsThreads) s_tot[threadIdx.x] = 0u;
+    if (threadIdx.x == 0) s_first = blocks <= kCsThreads ? 0u : max(k / (uint32_t)kCsBlockCells, 128u) - 128u;
+    __syncthreads();
+    const uint32_t first_block = s_first;
     const uint32_t kp = __shfl_up(k, 1, 64);
     const bool head = valid && (lane == 0 || kp != k);
     const uint64_t heads = __ballot(head);
     const uint64_t vmask = __ballot(valid);   // a prefix of the lanes
+    // the total of the key's block: one addition for a wavefront in one block
+    const uint32_t blk = k / (uint32_t)kCsBlockCells;
+    const bool same = !__any(valid && blk != (uint32_t)__builtin_amdgcn_readfirstlane((int)blk));
+    auto add = [&](uint32_t v) {
+        if (blk - first_block < (uint32_t)kCsThreads) atomicAdd(&s_tot[blk - first_block], v);
+        else atomicAdd(&bsum[kCopies * blk + blockIdx.x % kCopies], v);
+    };
     uint32_t base = 0;
     if (head) {
         const uint64_t after = lane == 63 ? 0ull : (heads >> (lane + 1));
         const int next = after ? lane + __ffsll((unsigned long long)after) : __popcll(vmask);
-        base = atomicAdd(&cnt[k], (uint32_t)(next - lane));
-        used[k / (uint32_t)kCsBlockCells] = 1u;
+        const uint32_t run = (uint32_t)(next - lane);
+        base = atomicAdd(&cnt[k], run);
+        if (!same) add(run);
     }
+    if (same && valid && lane == 0) add((uint32_t)__popcll(vmask));
 
     // the run's head: highest head lane at or below this lane
     const uint64_t upto = heads & (lane == 63 ? ~0ull : ((2ull << lane) - 1));
     const int hl = upto ? 63 - __clzll((long long)upto) : 0;
     const uint32_t b = __shfl(base, hl, 64);
     if (valid) rank[i] = b + (uint32_t)(lane - hl);
+    __syncthreads();
+    const uint32_t tot = threadIdx.x < kCsThreads ? s_tot[threadIdx.x] : 0u;
+    if (tot) atomicAdd(&bsum[kCopies * (first_block + threadIdx.x) + blockIdx.x % kCopies], tot);
 }
 
 // The 16 counts of this thread (cells base .. base + 15, zero past the end).
@@ -113,39 +149,23 @@ __device__ __forceinline__ uint32_t block_scan(uint32_t v, uint32_t* s_wave, uin
     return off + x - v;
 }
 
-__global__ __launch_bounds__(kCsThreads) void k_cs_reduce(const uint32_t* __restrict__ cnt, uint32_t cells,
-                                                          const uint32_t* __restrict__ used,
-                                                          uint32_t* __restrict__ bsum) {
-    __shared__ uint32_t s_wave[kCsThreads / 64];
-    if (!used[blockIdx.x]) {   // the same for the whole workgroup
-        if (threadIdx.x == 0) bsum[blockIdx.x] = 0u;
-        return;
-    }
-    const uint32_t base = blockIdx.x * (uint32_t)kCsBlockCells + threadIdx.x * (uint32_t)kCsPerThread;
-    uint32_t c[kCsPerThread];
-    load16(cnt, cells, base, c);
-    uint32_t s = 0;
-#pragma unroll
-    for (int j = 0; j < kCsPerThread; ++j) s += c[j];
-    uint32_t tot;
-    (void)block_scan(s, s_wave, &tot);
-    if (threadIdx.x == 0) bsum[blockIdx.x] = tot;
-}
-
 __global__ __launch_bounds__(kCsThreads) void k_cs_ranges(uint32_t* __restrict__ cnt, uint32_t cells,
                                                           const uint32_t* __restrict__ bsum,
-                                                          uint32_t* __restrict__ used,
                                                           int2* __restrict__ range) {
     __shared__ uint32_t s_wave[kCsThreads / 64];
-    // every thread reads the flag before the scans' barriers; thread 0
-    // clears it after them
-    if (!used[blockIdx.x]) return;   // no occupied cell in the block
+    static_assert(kCopies == 8, "two vectors a block");
+    const uint4* const totals = reinterpret_cast<const uint4*>(bsum);
+    auto any4 = [](uint4 v) { return v.x | v.y | v.z | v.w; };
+    if (!(any4(totals[2 * blockIdx.x]) | any4(totals[2 * blockIdx.x + 1]))) return;   // no occupied cell in the block
     const uint32_t base = blockIdx.x * (uint32_t)kCsBlockCells + threadIdx.x * (uint32_t)kCsPerThread;
     uint32_t c[kCsPerThread];
     load16(cnt, cells, base, c);
     // offset of this block: the totals of the blocks before it
     uint32_t before = 0;
-    for (uint32_t j = threadIdx.x; j < blockIdx.x; j += kCsThreads) before += bsum[j];
+    for (uint32_t j = threadIdx.x; j < 2 * blockIdx.x; j += kCsThreads) {
+        const uint4 v = totals[j];
+        before += v.x + v.y + v.z + v.w;
+    }
     uint32_t off;
     (void)block_scan(before, s_wave, &off);
     uint32_t s = 0;
@@ -161,16 +181,17 @@ __global__ __launch_bounds__(kCsThreads) void k_cs_ranges(uint32_t* __restrict__
         }
         start += c[j];
     }
-    if (threadIdx.x == 0) used[blockIdx.x] = 0u;
 }
 
 __global__ __launch_bounds__(kCsThreads) void k_cs_scatter(const uint32_t* __restrict__ keys, uint32_t n_host,
                                                            const uint32_t* __restrict__ n_dev,
                                                            const uint32_t* __restrict__ rank,
                                                            const int2* __restrict__ range,
-                                                           uint32_t* __restrict__ skey, uint32_t* __restrict__ perm) {
+                                                           uint32_t* __restrict__ skey, uint32_t* __restrict__ perm,
+                                                           uint32_t* __restrict__ bsum, uint32_t blocks) {
     const uint32_t n = n_dev ? *n_dev : n_host;
     uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    for (uint32_t j = i; j < kCopies * blocks; j += gridDim.x * blockDim.x) bsum[j] = 0u;
     if (i >= n) return;
     const uint32_t k = keys[i];
     const uint32_t d = (uint32_t)range[k].x + rank[i];
@@ -179,6 +200,7 @@ __global__ __launch_bounds__(kCsThreads) void k_cs_scatter(const uint32_t* __res
 }
 
 inline unsigned grid_for(uint32_t n) { return (n + kCsThreads - 1) / kCsThreads; }
+inline unsigned count_grid(uint32_t n) { return (n + kCountThreads - 1) / kCountThreads; }
 
 }  // namespace
 
@@ -192,11 +214,10 @@ hipError_t CellSort::init(uint32_t ncells, uint32_t capacity) {
     const size_t padded = (size_t)blocks * kCsBlockCells;
     if ((e = hipMalloc(&cnt, sizeof(uint32_t) * (padded ? padded : 1))) != hipSuccess) return e;
     if ((e = hipMalloc(&rank, sizeof(uint32_t) * (capacity ? capacity : 1))) != hipSuccess) return e;
-    if ((e = hipMalloc(&bsum, sizeof(uint32_t) * (blocks ? blocks : 1))) != hipSuccess) return e;
-    if ((e = hipMalloc(&used, sizeof(uint32_t) * (blocks ? blocks : 1))) != hipSuccess) return e;
+    if ((e = hipMalloc(&bsum, sizeof(uint32_t) * kCopies * (blocks ? blocks : 1))) != hipSuccess) return e;
     if ((e = hipMemset(cnt, 0, sizeof(uint32_t) * (padded ? padded : 1))) != hipSuccess) return e;
-    if ((e = hipMemset(used, 0, sizeof(uint32_t) * (blocks ? blocks : 1))) != hipSuccess) return e;
-    bytes = sizeof(uint32_t) * (padded + capacity + 2 * blocks);
+    if ((e = hipMemset(bsum, 0, sizeof(uint32_t) * kCopies * (blocks ? blocks : 1))) != hipSuccess) return e;
+    bytes = sizeof(uint32_t) * (padded + capacity + kCopies * blocks);
     return hipDeviceSynchronize();
 }
 
@@ -204,31 +225,40 @@ void CellSort::release() {
     if (cnt) (void)hipFree(cnt);
     if (rank) (void)hipFree(rank);
     if (bsum) (void)hipFree(bsum);
-    if (used) (void)hipFree(used);
-    cnt = rank = bsum = used = nullptr;
+    cnt = rank = bsum = nullptr;
     bytes = 0;
 }
 
 void CellSort::sort(hipStream_t st, const uint32_t* keys, uint32_t n, uint32_t* skey, uint32_t* perm,
                     int2* range, bool clear_prev) {
     if (n == 0) return;
-    launch(st, keys, n, nullptr, n, skey, perm, range, clear_prev ? skey : nullptr, n);
+    hipLaunchKernelGGL(k_cs_count<false>, dim3(count_grid(n)), dim3(kCountThreads), 0, st, KeysFirst(),
+                       const_cast<uint32_t*>(keys), n, nullptr, cnt, rank, bsum, blocks, clear_prev ? skey : nullptr,
+                       n, range);
+    finish(st, keys, n, nullptr, n, skey, perm, range);
+}
+
+void CellSort::sort_first(hipStream_t st, const KeysFirst& first, uint32_t* keys, uint32_t n, uint32_t* skey,
+                          uint32_t* perm, int2* range) {
+    if (n == 0) return;
+    hipLaunchKernelGGL(k_cs_count<true>, dim3(count_grid(n)), dim3(kCountThreads), 0, st, first, keys, n, nullptr, cnt,
+                       rank, bsum, blocks, nullptr, 0u, range);
+    finish(st, keys, n, nullptr, n, skey, perm, range);
 }
 
 void CellSort::sort(hipStream_t st, const uint32_t* keys, const uint32_t* n_dev, uint32_t capacity, uint32_t* skey,
                     uint32_t* perm, int2* range) {
     if (capacity == 0) return;
-    launch(st, keys, 0, n_dev, capacity, skey, perm, range, nullptr, 0);
+    hipLaunchKernelGGL(k_cs_count<false>, dim3(count_grid(capacity)), dim3(kCountThreads), 0, st, KeysFirst(),
+                       const_cast<uint32_t*>(keys), 0u, n_dev, cnt, rank, bsum, blocks, nullptr, 0u, range);
+    finish(st, keys, 0, n_dev, capacity, skey, perm, range);
 }
 
-void CellSort::launch(hipStream_t st, const uint32_t* keys, uint32_t n, const uint32_t* n_dev, uint32_t grid_n,
-                      uint32_t* skey, uint32_t* perm, int2* range, const uint32_t* prev_skey, uint32_t prev_n) {
-    hipLaunchKernelGGL(k_cs_count, dim3(grid_for(grid_n)), dim3(kCsThreads), 0, st, keys, n, n_dev, cnt, rank,
-                       used, prev_skey, prev_n, range);
-    hipLaunchKernelGGL(k_cs_reduce, dim3(blocks), dim3(kCsThreads), 0, st, cnt, cells, used, bsum);
-    hipLaunchKernelGGL(k_cs_ranges, dim3(blocks), dim3(kCsThreads), 0, st, cnt, cells, bsum, used, range);
+void CellSort::finish(hipStream_t st, const uint32_t* keys, uint32_t n, const uint32_t* n_dev, uint32_t grid_n,
+                      uint32_t* skey, uint32_t* perm, int2* range) {
+    hipLaunchKernelGGL(k_cs_ranges, dim3(blocks), dim3(kCsThreads), 0, st, cnt, cells, bsum, range);
     hipLaunchKernelGGL(k_cs_scatter, dim3(grid_for(grid_n)), dim3(kCsThreads), 0, st, keys, n, n_dev, rank, range,
-                       skey, perm);
+                       skey, perm, bsum, blocks);
 }
 
 }  // namespace sph

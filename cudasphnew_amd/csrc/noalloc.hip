@@ -8,7 +8,7 @@
 // object: each GPU the library runs on holds its own copy until the process
 // ends, at the address hipGetSymbolAddress returns with that device current.
 // Calls on one GPU share it; each call clears what must start cleared (the
-// cell table, the counting sort's counts and block flags), so a call does
+// cell table, the counting sort's counts and totals), so a call does
 // not depend on the last one's contents, but calls that overlap on one GPU
 // (two streams, two host threads) race on it.
 #include <algorithm>
@@ -51,8 +51,7 @@ struct Layout {
     // counts padded to whole count blocks (the sort reads them as vectors)
     static constexpr size_t cnt = range + align256(sizeof(int2) * (size_t)kNaMaxCells);
     static constexpr size_t bsum = cnt + align256(sizeof(uint32_t) * (size_t)kNaMaxBlocks * kNaCountBlock);
-    static constexpr size_t used = bsum + align256(sizeof(uint32_t) * (size_t)kNaMaxBlocks);
-    static constexpr size_t masks = used + align256(sizeof(uint32_t) * (size_t)kNaMaxBlocks);
+    static constexpr size_t masks = bsum + align256(sizeof(uint32_t) * kCsCopies * (size_t)kNaMaxBlocks);
     static constexpr size_t bytes = masks + align256(sizeof(uint64_t) * row_words_u64(kNaMaxParticles));
 };
 static_assert(Layout::bytes == SPH_NOALLOC_SCRATCH_BYTES, "scratch size differs from the header's figure");
@@ -79,13 +78,13 @@ hipError_t scratch_address(int dev, unsigned char** out) {
 constexpr int kNaThreads = 256;
 
 // Per call of the counting-sort path: the scene record, the slot range, a
-// cleared status word, an empty cell table, zero counts and block flags, and
+// cleared status word, an empty cell table, zero counts and block totals, and
 // the original ids (the indices; the first step reads the caller's arrays).
 __global__ __launch_bounds__(kNaThreads) void k_na_init(DevScene S, DevScene* __restrict__ d_scene,
                                                         uint32_t* __restrict__ begins, uint32_t* __restrict__ status,
                                                         uint32_t n, uint32_t ncells, uint32_t ncount,
                                                         uint32_t nblocks, int2* __restrict__ range,
-                                                        uint32_t* __restrict__ cnt, uint32_t* __restrict__ used,
+                                                        uint32_t* __restrict__ cnt, uint32_t* __restrict__ bsum,
                                                         uint32_t* __restrict__ oid_a) {
     const uint32_t stride = gridDim.x * blockDim.x;
     const uint32_t t0 = blockIdx.x * blockDim.x + threadIdx.x;
@@ -97,7 +96,7 @@ __global__ __launch_bounds__(kNaThreads) void k_na_init(DevScene S, DevScene* __
     }
     for (uint32_t i = t0; i < ncells; i += stride) range[i] = make_int2(-1, -1);
     for (uint32_t i = t0; i < ncount; i += stride) cnt[i] = 0u;
-    for (uint32_t i = t0; i < nblocks; i += stride) used[i] = 0u;
+    for (uint32_t i = t0; i < kCsCopies * nblocks; i += stride) bsum[i] = 0u;
     for (uint32_t i = t0; i < n; i += stride) oid_a[i] = i;
 }
 
@@ -193,7 +192,6 @@ extern "C" sph_status sph_step_noalloc(const sph_params* P, const sph_device_bou
     cs.cnt = reinterpret_cast<uint32_t*>(base + Layout::cnt);
     cs.rank = reinterpret_cast<uint32_t*>(base + Layout::rank);
     cs.bsum = reinterpret_cast<uint32_t*>(base + Layout::bsum);
-    cs.used = reinterpret_cast<uint32_t*>(base + Layout::used);
 
     // The first step reads the caller's particles, the last one returns them
     // there by id (no copies in and out: 7 us a call).  A small set sorts in
@@ -207,7 +205,7 @@ extern "C" sph_status sph_step_noalloc(const sph_params* P, const sph_device_bou
         hipLaunchKernelGGL(k_na_init, dim3(init_grid), dim3(kNaThreads), 0, st, S,
                            reinterpret_cast<DevScene*>(base + Layout::scene),
                            reinterpret_cast<uint32_t*>(base + Layout::begins), b.status, n, (uint32_t)cells, ncount,
-                           cs.blocks, b.range, cs.cnt, cs.used, b.oid_a);
+                           cs.blocks, b.range, cs.cnt, cs.bsum, b.oid_a);
     }
     float4* const own_pos = b.pos_a;
     float4* const own_vel = b.vel_a;
@@ -226,8 +224,15 @@ extern "C" sph_status sph_step_noalloc(const sph_params* P, const sph_device_bou
             }
             launch_small_sort(st, b, (uint32_t)cells, S, f);
         } else {
-            if (first) launch_hash(st, b);
-            cs.sort(st, b.key, n, b.skey, b.perm, b.range, !first);
+            if (first) {
+                KeysFirst f;
+                f.scene = S;
+                f.pos = b.pos_a;
+                f.status = b.status;
+                cs.sort_first(st, f, b.key, n, b.skey, b.perm, b.range);
+            } else {
+                cs.sort(st, b.key, n, b.skey, b.perm, b.range, true);
+            }
             launch_reorder(st, b);
         }
         launch_density(st, b, 1);

@@ -771,7 +771,7 @@ sph_status sph_boundary_map_load(const char* path, sph_boundary_map_config* cfg,
  * original id, bit for bit. */
 #define SPH_NOALLOC_MAX_PARTICLES 262144u
 #define SPH_NOALLOC_MAX_CELLS 1048576u
-#define SPH_NOALLOC_SCRATCH_BYTES 87034880u
+#define SPH_NOALLOC_SCRATCH_BYTES 87041024u
 typedef struct sph_device_boundary {
     float origin[3];
     float spacing;
