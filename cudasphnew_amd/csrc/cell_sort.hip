@@ -5,7 +5,10 @@
 //                 and the totals of 4096-cell blocks, added up in LDS per
 //                 workgroup of 1,024 first and then in one of eight copies
 //                 (workgroups of 256 and a single copy serialise: 8.2 us in
-//                 place of 4.9 at 250,000 particles, 9.4 and 6.9 at 1M)
+//                 place of 4.9 at 250,000 particles, 9.4 and 6.9 at 1M), with a
+//                 window of 1,024 blocks (256 leave the totals of particles in
+//                 no cell order to global memory: 10.6 in place of 4.8 for the
+//                 sub-particles of a two-scale step)
 //   k_cs_ranges   cell starts = offset of the block (sum of the totals of
 //                 the blocks before it, read by the whole workgroup) + scan
 //                 inside the block (16 counts per thread, read as four 16-byte
@@ -47,8 +50,8 @@ __global__ __launch_bounds__(kCountThreads) void k_cs_count(KeysFirst first, uin
                                                          uint32_t* __restrict__ bsum, uint32_t blocks,
                                                          const uint32_t* __restrict__ prev_skey, uint32_t prev_n,
                                                          int2* __restrict__ range) {
-    // totals of the kCsThreads blocks from `first_block` on
-    __shared__ uint32_t s_tot[kCsThreads];
+    // totals of the kCountThreads blocks from `first_block` on
+    __shared__ uint32_t s_tot[kCountThreads];
     __shared__ uint32_t s_first;
     const uint32_t n = n_dev ? *n_dev : n_host;
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -72,8 +75,8 @@ __global__ __launch_bounds__(kCountThreads) void k_cs_count(KeysFirst first, uin
             k = keys[i];
         }
     }
-    if (threadIdx.x < kCsThreads) s_tot[threadIdx.x] = 0u;
-    if (threadIdx.x == 0) s_first = blocks <= kCsThreads ? 0u : max(k / (uint32_t)kCsBlockCells, 128u) - 128u;
+    s_tot[threadIdx.x] = 0u;
+    if (threadIdx.x == 0) s_first = blocks <= kCountThreads ? 0u : max(k / (uint32_t)kCsBlockCells, 512u) - 512u;
     __syncthreads();
     const uint32_t first_block = s_first;
     const uint32_t kp = __shfl_up(k, 1, 64);
@@ -84,7 +87,7 @@ __global__ __launch_bounds__(kCountThreads) void k_cs_count(KeysFirst first, uin
     const uint32_t blk = k / (uint32_t)kCsBlockCells;
     const bool same = !__any(valid && blk != (uint32_t)__builtin_amdgcn_readfirstlane((int)blk));
     auto add = [&](uint32_t v) {
-        if (blk - first_block < (uint32_t)kCsThreads) atomicAdd(&s_tot[blk - first_block], v);
+        if (blk - first_block < (uint32_t)kCountThreads) atomicAdd(&s_tot[blk - first_block], v);
         else atomicAdd(&bsum[kCopies * blk + blockIdx.x % kCopies], v);
     };
     uint32_t base = 0;
@@ -103,7 +106,7 @@ __global__ __launch_bounds__(kCountThreads) void k_cs_count(KeysFirst first, uin
     const uint32_t b = __shfl(base, hl, 64);
     if (valid) rank[i] = b + (uint32_t)(lane - hl);
     __syncthreads();
-    const uint32_t tot = threadIdx.x < kCsThreads ? s_tot[threadIdx.x] : 0u;
+    const uint32_t tot = s_tot[threadIdx.x];
     if (tot) atomicAdd(&bsum[kCopies * (first_block + threadIdx.x) + blockIdx.x % kCopies], tot);
 }
 

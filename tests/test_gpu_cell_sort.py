@@ -1,7 +1,7 @@
 """The counting sort's block totals (csrc/cell_sort.hip) on a key space wider
-than the window of blocks a workgroup adds up in LDS (256 of 4,096 cells):
-keys, ids and cell ranges equal the oracle's, from shuffled particles (most
-totals outside the window) and from the sorted ones of the next step."""
+than the window of blocks a workgroup adds up in LDS (1,024 of 4,096 cells):
+keys, ids and cell ranges equal the oracle's, from shuffled particles (of
+the wider grid some outside the window) and from the sorted ones of the next step."""
 import numpy as np
 import pytest
 
@@ -11,7 +11,7 @@ from tests.test_gpu_parity import _check_sort
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("grid,n", [((200, 200, 40), 101001), ((131, 100, 81), 70000)])   # 391 and 260 blocks
+@pytest.mark.parametrize("grid,n", [((200, 200, 40), 101001), ((170, 160, 160), 280000)])   # 391, 1,063 blocks
 def test_wide_key_space(grid, n):
     base = S.make_scene("dam16k")
     p = base.params
