@@ -851,7 +851,12 @@ __device__ __forceinline__ void net_cd_normal(const NetView& net, float4 x, floa
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 float sc;
-                g[j][a] += (float)sgn * decode(net, y[j], sc) * inv2s;
+                const float v = (float)sgn * decode(net, y[j], sc) * inv2s;
+                // selects: an index known only at run time would put g in
+                // scratch memory
+                g[j][0] = a == 0 ? g[j][0] + v : g[j][0];
+                g[j][1] = a == 1 ? g[j][1] + v : g[j][1];
+                g[j][2] = a == 2 ? g[j][2] + v : g[j][2];
             }
         }
 }
@@ -944,13 +949,14 @@ __global__ __launch_bounds__(kThreads) void k_wall_mlp(const uint2* __restrict__
     const uint32_t* L = list + S.p_begin;
     const uint32_t k = k0 + 16 * w + (lane & 15);
     const float4 x = pos[L[k < count ? k : k0]];
-    const NetView net = nets[t.x];
+    const NetView& net = nets[t.x];   // a copy would be scratch memory (its arrays are indexed)
     float g[4][3];
     net_cd_normal(net, x, S.bspacing, lane, w, sA1, sA2, g);
     if ((lane & 15) < 4) {
         const int j = lane & 15;
         const uint32_t kj = k0 + 16 * w + 4 * (lane >> 4) + j;
-        if (kj < count) rec[L[kj]] = make_float4(g[j][0], g[j][1], g[j][2], 0.0f);
+        auto own = [&](int c) { return j < 2 ? (j == 0 ? g[0][c] : g[1][c]) : (j == 2 ? g[2][c] : g[3][c]); };
+        if (kj < count) rec[L[kj]] = make_float4(own(0), own(1), own(2), 0.0f);
     }
 }
 

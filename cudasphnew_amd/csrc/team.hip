@@ -38,9 +38,15 @@ __device__ __forceinline__ void wave_sync() {
 }
 
 // The nine rows' runs of a team's particle: lane r < 9 finds row r, then all
-// lanes hold all rows.
+// lanes hold all rows.  b and cnt are indexed with constants only (a loop
+// over them that stays a loop puts both in scratch memory); row(r) asks lane r.
 struct TeamRows {
     int b[9], cnt[9];
+    int own_b, own_cnt;
+    __device__ __forceinline__ void row(int r, int& rb, int& rcnt) const {
+        rb = __shfl(own_b, r, kTeam);
+        rcnt = __shfl(own_cnt, r, kTeam);
+    }
 };
 
 __device__ __forceinline__ TeamRows team_rows(const int2* __restrict__ range, const DevScene& S, float4 xi, int c) {
@@ -48,10 +54,12 @@ __device__ __forceinline__ TeamRows team_rows(const int2* __restrict__ range, co
     int b = 0, e = 0;
     if (c < 9) row_slots(range, S, R, c / 3, c % 3, xi, b, e);
     TeamRows t;
+    t.own_b = b;
+    t.own_cnt = e - b;
 #pragma unroll
     for (int r = 0; r < 9; ++r) {
         t.b[r] = __shfl(b, r, kTeam);
-        t.cnt[r] = __shfl(e - b, r, kTeam);
+        t.cnt[r] = __shfl(t.own_cnt, r, kTeam);
     }
     return t;
 }
@@ -145,7 +153,8 @@ __global__ __launch_bounds__(kBlock) void k_density_team(const float4* __restric
         // 16 might not fit
 #pragma unroll 1
         for (int r = 0; r < 9; ++r) {
-            const int b = T.b[r], cnt = T.cnt[r];
+            int b, cnt;
+            T.row(r, b, cnt);
             for (int t0 = 0; __any(t0 < cnt); t0 += kTeam) {
                 const bool in = t0 + c < cnt;
                 const float4 xj = pos[in ? (uint32_t)(b + t0 + c) : s];
@@ -269,7 +278,9 @@ __global__ __launch_bounds__(kBlock) void k_force_team(
             for (int k = 0; k < (MASKS ? 18 : 9); ++k) {
                 const int r = k % 9;
                 const bool late = k >= 9;
-                const int b = T.b[r], cnt = MASKS && late != (T.cnt[r] > kRowMaxCands) ? 0 : T.cnt[r];
+                int b, cnt;
+                T.row(r, b, cnt);
+                if (MASKS && late != (cnt > kRowMaxCands)) cnt = 0;
                 for (int t0 = 0; __any(t0 < cnt); t0 += kTeam) {
                     const bool in = t0 + c < cnt;
                     const uint32_t q = in ? (uint32_t)(b + t0 + c) : s;
