@@ -104,8 +104,9 @@ struct Engine {
     // graph capture of the steady-state step, plain and two-scale
     bool use_graph = false;
     uint32_t retune_every = 0;   // re-run the autotuner before every n-th step (0: never)
-    hipGraph_t graph = nullptr;
-    hipGraphExec_t graph_exec = nullptr;
+    static constexpr int kGraphSizes = 3;
+    hipGraph_t graph[kGraphSizes] = {};           // of 2^k steps
+    hipGraphExec_t graph_exec[kGraphSizes] = {};
 
     TwoScale* ts = nullptr;
     bool last_two_scale = false;
