@@ -581,16 +581,22 @@ __device__ __forceinline__ void sub_row_slots(const int2* __restrict__ srange, c
     const float dz = fmaxf(fmaxf(z0 - xi.z, xi.z - (z0 + S.cell_sub)), 0.0f);
     if ((dy * dy + dz * dz) * 0.99999f > S.h2_sub) return;
     const uint32_t rowbase = (uint32_t)(S.snx * (S.sny * k + j));
-    b = 0x7fffffff;
-    e = -1;
-    for (int i = R.lx; i <= R.hx; ++i) {
-        const int2 r = srange[rowbase + (uint32_t)i];
-        if (r.x >= 0) {
-            b = min(b, r.x);
-            e = max(e, r.y);
-        }
+    if (R.lx > R.hx) return;
+    // the run's first, second and last cell are read together; an empty one
+    // (-1, -1) drops out of the unsigned minimum and the signed maximum
+    const int2* __restrict__ row = srange + rowbase;
+    const int m = min(R.lx + 1, R.hx);
+    const int2 r0 = row[R.lx], r1 = row[m], r2 = row[R.hx];
+    uint32_t lo = min(min((uint32_t)r0.x, (uint32_t)r1.x), (uint32_t)r2.x);
+    int hi = max(max(r0.y, r1.y), r2.y);
+    for (int i = m + 1; i < R.hx; ++i) {   // a support of more than a cell
+        const int2 r = row[i];
+        lo = min(lo, (uint32_t)r.x);
+        hi = max(hi, r.y);
     }
-    if (e < b) { b = 0; e = 0; }
+    if (hi < 0) return;
+    b = (int)lo;
+    e = hi;
 }
 
 // Row words of the sub passes: the coarse pair's format (common.h) over the
@@ -619,11 +625,24 @@ __global__ __launch_bounds__(kB) void k_ts_density(const TSCounts* __restrict__ 
         float sum = 0.0f;
         const float4 xi = spos_s[t];
         const F4Buf sp(spos_s);
-        const SubRows R = sub_rows(S, xi);
+        // lane j finds the runs of rows j, j + 4 and j + 8: one round of table
+        // reads in place of one a row (30.7 -> 22.9 us for 111,000
+        // sub-particles; loading the next row's candidates early takes 42: the
+        // loads past a row's end cost more than the wait)
+        int rb[3], re[3];
+        {
+            const SubRows R = sub_rows(S, xi);
+#pragma unroll
+            for (int i = 0; i < 3; ++i) {
+                const int row = lane + kTsLanes * i;
+                rb[i] = re[i] = 0;
+                if (split && row < 9) sub_row_slots(srange, S, R, row / 3, row % 3, xi, rb[i], re[i]);
+            }
+        }
 #pragma unroll 1
         for (int row = 0; row < 9; ++row) {
-            int b = 0, e = 0;
-            if (split) sub_row_slots(srange, S, R, row / 3, row % 3, xi, b, e);
+            const int b = __shfl(row < 4 ? rb[0] : (row < 8 ? rb[1] : rb[2]), row % kTsLanes, kTsLanes);
+            const int e = __shfl(row < 4 ? re[0] : (row < 8 ? re[1] : re[2]), row % kTsLanes, kTsLanes);
             // the sign bits of h_sub^2 - r^2 of this lane's candidates
             // b + lane + 4k, newest in bit 0 (as in the coarse density pass)
             uint32_t far = 0;
@@ -672,18 +691,26 @@ __global__ __launch_bounds__(kB) void k_ts_density(const TSCounts* __restrict__ 
 // and the collision response for every sub-particle.  One thread per
 // sub-particle.  The pair terms run over the set bits of the density pass's
 // row words, in candidate order (rows in z-major, y-minor order, slots
-// ascending), so a wavefront executes them as often as its lane with the most
-// neighbours in the row; a row of more than kRowMaxCands candidates is tested
-// here.  (Before the rows kept chunks past 32 candidates, such rows were
+// ascending), expanded into a hit list in LDS as in the coarse force pass, so
+// a wavefront executes them as often as its lane with the most neighbours and
+// three gathers are in flight: there are two wavefronts a SIMD, and the pass is
+// bound by the latency of a lane's chain of gathers (24.5 us for 111,000
+// sub-particles one gather at a time, row by row; 14.4 now).  The rows of a
+// sub-particle with one of more than kRowMaxCands candidates are walked in
+// place.  (Before the rows kept chunks past 32 candidates, such rows were
 // tested here too: on the two-scale workload after ~1,000 steps, as the
-// flow compresses, this pass took 120 us against 44 us now.)
-__global__ __launch_bounds__(kB) void k_ts_force(TSCounts* __restrict__ cnt, const uint32_t* __restrict__ sperm,
+// flow compresses, this pass took 120 us against 44 us after.)
+constexpr int kTsForceB = 128;   // threads; the list takes 24 KiB
+constexpr int kTsCap = 48;
+
+__global__ __launch_bounds__(kTsForceB) void k_ts_force(TSCounts* __restrict__ cnt, const uint32_t* __restrict__ sperm,
                                                  const float4* __restrict__ spos_s, const float4* __restrict__ svel_s,
                                                  const int2* __restrict__ srange, const DevScene* __restrict__ scenes,
                                                  const uint64_t* __restrict__ smasks, uint32_t cap,
                                                  const float* __restrict__ gridd, float4* __restrict__ spos_out,
                                                  float4* __restrict__ svel_out, float4* __restrict__ sacc,
                                                  uint32_t* __restrict__ status) {
+    __shared__ int s_list[kTsCap][kTsForceB];   // one column per thread: no barrier needed
     uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
     const uint32_t nsub = cnt->nsub;
     if (t == 0) {
@@ -705,11 +732,9 @@ __global__ __launch_bounds__(kB) void k_ts_force(TSCounts* __restrict__ cnt, con
         const float kr0 = S.stiff * S.rho0;
         float fpx = 0, fpy = 0, fpz = 0, fvx = 0, fvy = 0, fvz = 0, cgx = 0, cgy = 0, cgz = 0, cl = 0;
         const F4Buf sp(spos_s), sv(svel_s);
-        auto pair = [&](int q) {
-            float4 xj = sp[q];
+        auto pair_of = [&](float4 xj, float4 vj) {
             float dx = xi.x - xj.x, dy = xi.y - xj.y, dz = xi.z - xj.z;
             float r2 = dx * dx + dy * dy + dz * dz;
-            float4 vj = sv[q];
             // a distinct sub at distance 0 contributes nothing (every term
             // carries 1/r or 1/rho_j, both taken as 0 there)
             const bool nz = r2 > 0.0f;
@@ -726,31 +751,102 @@ __global__ __launch_bounds__(kB) void k_ts_force(TSCounts* __restrict__ cnt, con
             cgx += wc * dx; cgy += wc * dy; cgz += wc * dz;
             cl += invj * qd * (3.0f * h2 - 7.0f * r2);
         };
+        auto pair = [&](int q) { pair_of(sp[q], sv[q]); };
         auto near = [&](int q) {
             const float4 xj = spos_s[q];
             const float dx = xi.x - xj.x, dy = xi.y - xj.y, dz = xi.z - xj.z;
             const float r2 = dx * dx + dy * dy + dz * dz;
             return r2 <= h2 && r2 > 0.0f;
         };
-#pragma unroll 1
-        for (int row = 0; row < 9; ++row) {
-            const uint64_t w = smasks[(size_t)row * cap + t];
-            if (w != kRowLong) {
-                const uint32_t last = row_last_chunk(w);
-                for (uint32_t ch = 0; ch <= last; ++ch) {
-                    const int b = (int)(row_first(w) + 32u * ch);
-                    uint32_t m = ch == 0 ? (uint32_t)w : chunk_masks(smasks, cap)[chunk_at(cap, ch, row, t)];
-                    while (m) {
-                        const int u = __ffs(m) - 1;
-                        m &= m - 1;
-                        pair(b + u);
+        // unexpanded hits: bits[row] = the rest of the current chunk's mask;
+        // chunk / last: current and last chunk of each row, 2 bits per row
+        uint32_t bits[9];
+        int first[9];
+        uint32_t chunk = 0, last = 0;
+        bool any_long = false;
+        {
+            uint64_t w[9];
+#pragma unroll
+            for (int row = 0; row < 9; ++row) w[row] = smasks[(size_t)row * cap + t];
+#pragma unroll
+            for (int row = 0; row < 9; ++row) {
+                any_long |= w[row] == kRowLong;
+                bits[row] = (uint32_t)w[row];
+                first[row] = (int)row_first(w[row]);
+                last |= row_last_chunk(w[row]) << (2 * row);
+            }
+        }
+        if (!any_long) {
+            const uint32_t* const cm = chunk_masks(smasks, cap);
+            const int tid = threadIdx.x;
+            int m;
+            do {
+                m = 0;
+#pragma unroll
+                for (int row = 0; row < 9; ++row) {
+                    for (;;) {
+                        const uint32_t c = chunk >> (2 * row) & 3u;
+                        const int b = first[row] + (int)(c << 5);
+                        uint32_t lo = bits[row];
+                        const int take = min((int)__popc(lo), kTsCap - m);
+                        for (int i = 0; i < take; ++i) {
+                            s_list[m + i][tid] = b + __builtin_ctz(lo);
+                            lo &= lo - 1;
+                        }
+                        m += take;
+                        bits[row] = lo;
+                        if (lo || c == (last >> (2 * row) & 3u)) break;
+                        chunk += 1u << (2 * row);   // next chunk of a long row
+                        bits[row] = cm[chunk_at(cap, c + 1, row, t)];
                     }
                 }
-            } else {
-                int b, e;
-                sub_row_slots(srange, S, sub_rows(S, xi), row / 3, row % 3, xi, b, e);
-                for (int q = b; q < e; ++q)
-                    if (near(q)) pair(q);
+                if (m > 0) {
+                    // three entries in flight; past the end the last one
+                    // repeats, loaded but not evaluated
+                    int q = s_list[0][tid];
+                    float4 x0 = sp[q], v0 = sv[q];
+                    q = s_list[min(1, m - 1)][tid];
+                    float4 x1 = sp[q], v1 = sv[q];
+                    q = s_list[min(2, m - 1)][tid];
+                    float4 x2 = sp[q], v2 = sv[q];
+                    int k = 0;
+                    for (; k + 3 < m; k += 3) {
+                        pair_of(x0, v0);
+                        q = s_list[k + 3][tid];
+                        x0 = sp[q]; v0 = sv[q];
+                        pair_of(x1, v1);
+                        q = s_list[min(k + 4, m - 1)][tid];
+                        x1 = sp[q]; v1 = sv[q];
+                        pair_of(x2, v2);
+                        q = s_list[min(k + 5, m - 1)][tid];
+                        x2 = sp[q]; v2 = sv[q];
+                    }
+                    pair_of(x0, v0);
+                    if (k + 1 < m) pair_of(x1, v1);
+                    if (k + 2 < m) pair_of(x2, v2);
+                }
+            } while (m == kTsCap);   // a full list: hits may remain
+        } else {
+#pragma unroll 1
+            for (int row = 0; row < 9; ++row) {
+                const uint64_t w = smasks[(size_t)row * cap + t];
+                if (w != kRowLong) {
+                    const uint32_t last = row_last_chunk(w);
+                    for (uint32_t ch = 0; ch <= last; ++ch) {
+                        const int b = (int)(row_first(w) + 32u * ch);
+                        uint32_t m = ch == 0 ? (uint32_t)w : chunk_masks(smasks, cap)[chunk_at(cap, ch, row, t)];
+                        while (m) {
+                            const int u = __ffs(m) - 1;
+                            m &= m - 1;
+                            pair(b + u);
+                        }
+                    }
+                } else {
+                    int b, e;
+                    sub_row_slots(srange, S, sub_rows(S, xi), row / 3, row % 3, xi, b, e);
+                    for (int q = b; q < e; ++q)
+                        if (near(q)) pair(q);
+                }
             }
         }
         const float cpf = -S.mass_sub * S.grad_spiky_sub, cvf = S.mu * S.mass_sub * S.lapl_visc_sub;
@@ -917,7 +1013,7 @@ static void sub_pass(Engine& e, TwoScale& t, bool keys_ready) {
     const unsigned sub_grid = (unsigned)std::min<uint64_t>(kTsGrid, ((uint64_t)t.cap * kTsLanes + kB - 1) / kB);
     hipLaunchKernelGGL(k_ts_density, dim3(sub_grid), dim3(kB), 0, st, t.counts, t.sperm, t.spos_s, t.svel_s,
                        t.srange, e.d_scenes, t.cap, t.smasks);
-    hipLaunchKernelGGL(k_ts_force, dim3(nblocks(t.cap)), dim3(kB), 0, st, t.counts, t.sperm, t.spos_s, t.svel_s,
+    hipLaunchKernelGGL(k_ts_force, dim3((t.cap + kTsForceB - 1) / kTsForceB), dim3(kTsForceB), 0, st, t.counts, t.sperm, t.spos_s, t.svel_s,
                        t.srange, e.d_scenes, t.smasks, t.cap, e.gridd, t.spos_out, t.svel_out, t.sacc, e.status);
     e.mark(kStageTwoScaleSubPhysics);
 }
