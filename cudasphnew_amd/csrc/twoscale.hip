@@ -240,29 +240,31 @@ __global__ __launch_bounds__(kB) void k_ts_mark_rows(const float4* __restrict__ 
     }
 }
 
-// The class of each particle by original id: 0 default, 1 split (split bit,
-// boundary bit set by itself), 2 boundary only.
-__global__ __launch_bounds__(kB) void k_ts_classify(const uint8_t* __restrict__ state_fin,
-                                                    const uint32_t* __restrict__ oid, uint32_t n,
-                                                    uint8_t* __restrict__ cls) {
-    uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= n) return;
-    const int c = state_fin[s] & 3;
-    cls[oid[s]] = c == 0 ? 0 : (c == 2 ? 2 : 1);
-}
-
-// 3-way compaction in original-id order: per-tile counts ...
-__global__ __launch_bounds__(kB) void k_ts_count(const uint8_t* __restrict__ cls, uint32_t n,
-                                                 uint32_t* __restrict__ blk, uint32_t nblk) {
+// 3-way compaction in original-id order.  The class of each particle by
+// original id (0 default, 1 split: split bit, boundary bit set by itself, 2
+// boundary only), and the counts per tile ...
+__global__ __launch_bounds__(kB) void k_ts_count(const uint8_t* __restrict__ state_fin,
+                                                 const uint32_t* __restrict__ slot_of_oid, uint32_t n,
+                                                 uint8_t* __restrict__ cls, uint32_t* __restrict__ blk,
+                                                 uint32_t nblk) {
     __shared__ uint32_t s_c[3];
     if (threadIdx.x < 3) s_c[threadIdx.x] = 0;
     __syncthreads();
-    uint32_t c[3] = {0, 0, 0};
-    uint32_t base = blockIdx.x * kCompactTile;
+    uint32_t split = 0, bound = 0, all = 0;
+    const uint32_t base = blockIdx.x * kCompactTile;
+#pragma unroll
     for (int r = 0; r < kCompactItems; ++r) {
-        uint32_t i = base + r * kB + threadIdx.x;
-        if (i < n) c[cls[i]]++;
+        const uint32_t i = base + r * kB + threadIdx.x;
+        if (i < n) {
+            const int f = state_fin[slot_of_oid[i]] & 3;
+            cls[i] = f == 0 ? 0 : (f == 2 ? 2 : 1);
+            ++all;
+            split += f & 1;
+            bound += f == 2;
+        }
     }
+    uint32_t c[3] = {all - split - bound, split, bound};
+#pragma unroll
     for (int t = 0; t < 3; ++t) {
         uint32_t v = c[t];
         for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
@@ -365,40 +367,14 @@ __global__ __launch_bounds__(kB) void k_ts_collect(const uint8_t* __restrict__ c
     }
 }
 
-// initialize_sub_particles for every split and boundary parent (cu:1023-
-// 1090): 8 children, directions (+-1,+-1,+-1) in the order of the reference
-// table (x sign from bit 2, y from bit 1, z from bit 0 of the child index).
-// The sub cell keys of the seeded positions (compute_sub_particle_hash,
-// cu:121-153) are computed here too, and (clear_prev) the cells of the
-// previous step's sorted sub keys are invalidated before the sub sort
-// writes this step's ranges (what k_ts_hash does for a sub-particle step).
-__global__ __launch_bounds__(kB) void k_ts_seed(const TSCounts* __restrict__ cnt,
-                                                const uint32_t* __restrict__ split_ids,
-                                                const uint32_t* __restrict__ boundary_ids,
-                                                const uint32_t* __restrict__ slot_of_oid,
-                                                const float4* __restrict__ pos, const float4* __restrict__ vel,
-                                                const DevScene* __restrict__ scenes, float4* __restrict__ spos,
-                                                float4* __restrict__ svel, uint32_t* __restrict__ sid,
-                                                uint32_t* __restrict__ skey, uint32_t* __restrict__ status,
-                                                int clear_prev, const uint32_t* __restrict__ sskey,
-                                                int2* __restrict__ srange) {
-    uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (clear_prev && k < cnt->nsub_prev) {
-        const uint32_t pc = sskey[k];
-        if (k == 0 || sskey[k - 1] != pc) srange[pc] = make_int2(-1, -1);
-    }
-    const uint32_t nsub = cnt->nsub, nsplit = cnt->nsplit;
-    if (k >= nsub) return;
-    const DevScene& S = scenes[0];
-    uint32_t q = k >> 3, c = k & 7;
-    uint32_t id = q < nsplit ? split_ids[q] : boundary_ids[q - nsplit];
-    uint32_t slot = slot_of_oid[id];
-    float4 xp = pos[slot];
-    float4 vp = vel[slot];
+// Child c of a parent at xp with density rho (initialize_sub_particles,
+// cu:1023-1090): 8 children, directions (+-1,+-1,+-1) in the order of the
+// reference table (x sign from bit 2, y from bit 1, z from bit 0 of c).
+__device__ __forceinline__ float4 child_position(const DevScene& S, float4 xp, float rho, uint32_t c) {
     float radius, dirf;
     if (S.sub_placement == 0) {
         // r = (3 m / (4 pi rho))^(1/3), along the cube diagonals
-        float radicand = 3.0f * S.mass / (4.0f * 3.14159265358979323846f * vp.w);
+        float radicand = 3.0f * S.mass / (4.0f * 3.14159265358979323846f * rho);
         radius = cbrtf(radicand);
         dirf = 0.577350269f;   // 1/sqrt(3) (cu:1025)
     } else {
@@ -407,13 +383,7 @@ __global__ __launch_bounds__(kB) void k_ts_seed(const TSCounts* __restrict__ cnt
     }
     float off = radius * dirf;
     float ox = (c & 4) ? -off : off, oy = (c & 2) ? -off : off, oz = (c & 1) ? -off : off;
-    const float4 xs = make_float4(xp.x + ox, xp.y + oy, xp.z + oz, 0.0f);
-    spos[k] = xs;
-    svel[k] = make_float4(vp.x, vp.y, vp.z, 0.0f);
-    sid[k] = 8u * id + c;
-    uint32_t flags = 0;
-    skey[k] = sub_cell_key(S, xs.x, xs.y, xs.z, flags);
-    if (flags) atomicOr(status, flags);
+    return make_float4(xp.x + ox, xp.y + oy, xp.z + oz, 0.0f);
 }
 
 // project_quantities (cu:570-622, 1328-1381): boundary sub-particles take the
@@ -433,6 +403,91 @@ __device__ __forceinline__ float proj_sum(float v) {
     return v;
 }
 
+// The projected density at xs; every lane of the group takes part and has it.
+__device__ __forceinline__ float project_density(const DevScene& S, float4 xs, int lane,
+                                                 const float4* __restrict__ pos, const float4* __restrict__ vel,
+                                                 const int2* __restrict__ range) {
+    const float hs = S.h_sub, hs2 = S.h2_sub;
+    const int lx = range_coord(xs.x, -hs, S.ox, S.cell, S.nx), hx = range_coord(xs.x, hs, S.ox, S.cell, S.nx);
+    const int ly = range_coord(xs.y, -hs, S.oy, S.cell, S.ny), hy = range_coord(xs.y, hs, S.oy, S.cell, S.ny);
+    const int lz = range_coord(xs.z, -hs, S.oz, S.cell, S.nz), hz = range_coord(xs.z, hs, S.oz, S.cell, S.nz);
+    float sum = 0.0f, cntn = 0.0f;
+    if (hx >= lx && hy >= ly && hz >= lz) {   // else a range wrapped by the grid's "% dim": no cells
+        const int nxc = hx - lx + 1, nyc = hy - ly + 1, ncell = nxc * nyc * (hz - lz + 1);
+        for (int c = lane; c < ncell; c += kProjLanes) {
+            const int i = lx + c % nxc, j = ly + (c / nxc) % nyc, kk = lz + c / (nxc * nyc);
+            const int2 r = range[S.cell_offset + (uint32_t)(S.nx * (S.ny * kk + j) + i)];
+            for (int q = r.x; q < r.y; ++q) {
+                const float4 xj = pos[q];
+                const float dx = xs.x - xj.x, dy = xs.y - xj.y, dz = xs.z - xj.z;
+                if (dx * dx + dy * dy + dz * dz <= hs2) {
+                    sum += vel[q].w;
+                    cntn += 1.0f;
+                }
+            }
+        }
+    }
+    sum = proj_sum(sum);
+    cntn = proj_sum(cntn);
+    return cntn > 0.0f ? sum / cntn : S.rho0;
+}
+
+// The children of every split and boundary parent, and the projected density
+// of the boundary ones (blocks below kProjGrid: a group of lanes per boundary
+// child; it forms the child's position itself, so that the two parts need
+// no launch between them: 4.5 and 12.6 us one after the other, 14.2 together).  The sub
+// cell keys of the seeded positions (compute_sub_particle_hash, cu:121-153) are
+// computed here too, and (clear_prev) the cells of the previous step's sorted
+// sub keys are invalidated before the sub sort writes this step's ranges
+// (what k_ts_hash does for a sub-particle step).
+__global__ __launch_bounds__(kB) void k_ts_seed(const TSCounts* __restrict__ cnt,
+                                                const uint32_t* __restrict__ split_ids,
+                                                const uint32_t* __restrict__ boundary_ids,
+                                                const uint32_t* __restrict__ slot_of_oid,
+                                                const float4* __restrict__ pos, const float4* __restrict__ vel,
+                                                const int2* __restrict__ range,
+                                                const DevScene* __restrict__ scenes, float4* __restrict__ spos,
+                                                float4* __restrict__ svel, uint32_t* __restrict__ sid,
+                                                uint32_t* __restrict__ skey, uint32_t* __restrict__ status,
+                                                int clear_prev, const uint32_t* __restrict__ sskey,
+                                                int2* __restrict__ srange) {
+    const uint32_t nsub = cnt->nsub, nsplit = cnt->nsplit;
+    const DevScene& S = scenes[0];
+    if (blockIdx.x < kProjGrid) {
+        const uint32_t first = 8u * nsplit;
+        const uint64_t total = (uint64_t)(nsub > first ? nsub - first : 0u) * kProjLanes;
+        const uint64_t stride = (uint64_t)kProjGrid * kB;   // a multiple of kProjLanes
+        for (uint64_t g = (uint64_t)blockIdx.x * kB + threadIdx.x; g < total; g += stride) {
+            const uint32_t k = first + (uint32_t)(g / kProjLanes);
+            const uint32_t slot = slot_of_oid[boundary_ids[(k >> 3) - nsplit]];
+            const float4 vp = vel[slot];
+            const float4 xs = child_position(S, pos[slot], vp.w, k & 7);
+            const int lane = (int)(g % kProjLanes);
+            const float rho = project_density(S, xs, lane, pos, vel, range);
+            if (lane == 0) svel[k] = make_float4(vp.x, vp.y, vp.z, rho);
+        }
+        return;
+    }
+    const uint32_t k = (blockIdx.x - kProjGrid) * kB + threadIdx.x;
+    if (clear_prev && k < cnt->nsub_prev) {
+        const uint32_t pc = sskey[k];
+        if (k == 0 || sskey[k - 1] != pc) srange[pc] = make_int2(-1, -1);
+    }
+    if (k >= nsub) return;
+    uint32_t q = k >> 3, c = k & 7;
+    uint32_t id = q < nsplit ? split_ids[q] : boundary_ids[q - nsplit];
+    uint32_t slot = slot_of_oid[id];
+    float4 vp = vel[slot];
+    const float4 xs = child_position(S, pos[slot], vp.w, c);
+    spos[k] = xs;
+    if (q < nsplit) svel[k] = make_float4(vp.x, vp.y, vp.z, 0.0f);
+    sid[k] = 8u * id + c;
+    uint32_t flags = 0;
+    skey[k] = sub_cell_key(S, xs.x, xs.y, xs.z, flags);
+    if (flags) atomicOr(status, flags);
+}
+
+// The projection alone (a sub-particle step keeps its children).
 __global__ __launch_bounds__(kB) void k_ts_project(const TSCounts* __restrict__ cnt, const float4* __restrict__ spos,
                                                    float4* __restrict__ svel, const float4* __restrict__ pos,
                                                    const float4* __restrict__ vel, const int2* __restrict__ range,
@@ -440,34 +495,11 @@ __global__ __launch_bounds__(kB) void k_ts_project(const TSCounts* __restrict__ 
     const uint32_t nsub = cnt->nsub, first = 8u * cnt->nsplit;
     const uint64_t total = (uint64_t)(nsub > first ? nsub - first : 0u) * kProjLanes;
     const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;   // a multiple of kProjLanes
-    const DevScene& S = scenes[0];
-    const float hs = S.h_sub, hs2 = S.h2_sub;
     for (uint64_t g = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; g < total; g += stride) {
         const uint32_t k = first + (uint32_t)(g / kProjLanes);
         const int lane = (int)(g % kProjLanes);
-        const float4 xs = spos[k];
-        const int lx = range_coord(xs.x, -hs, S.ox, S.cell, S.nx), hx = range_coord(xs.x, hs, S.ox, S.cell, S.nx);
-        const int ly = range_coord(xs.y, -hs, S.oy, S.cell, S.ny), hy = range_coord(xs.y, hs, S.oy, S.cell, S.ny);
-        const int lz = range_coord(xs.z, -hs, S.oz, S.cell, S.nz), hz = range_coord(xs.z, hs, S.oz, S.cell, S.nz);
-        float sum = 0.0f, cntn = 0.0f;
-        if (hx >= lx && hy >= ly && hz >= lz) {   // else a range wrapped by the grid's "% dim": no cells
-            const int nxc = hx - lx + 1, nyc = hy - ly + 1, ncell = nxc * nyc * (hz - lz + 1);
-            for (int c = lane; c < ncell; c += kProjLanes) {
-                const int i = lx + c % nxc, j = ly + (c / nxc) % nyc, kk = lz + c / (nxc * nyc);
-                const int2 r = range[S.cell_offset + (uint32_t)(S.nx * (S.ny * kk + j) + i)];
-                for (int q = r.x; q < r.y; ++q) {
-                    const float4 xj = pos[q];
-                    const float dx = xs.x - xj.x, dy = xs.y - xj.y, dz = xs.z - xj.z;
-                    if (dx * dx + dy * dy + dz * dz <= hs2) {
-                        sum += vel[q].w;
-                        cntn += 1.0f;
-                    }
-                }
-            }
-        }
-        sum = proj_sum(sum);     // every lane of the group takes part
-        cntn = proj_sum(cntn);
-        if (lane == 0) svel[k].w = cntn > 0.0f ? sum / cntn : S.rho0;
+        const float rho = project_density(scenes[0], spos[k], lane, pos, vel, range);
+        if (lane == 0) svel[k].w = rho;
     }
 }
 
@@ -1037,17 +1069,14 @@ void twoscale_enqueue(Engine& e, const uint64_t* masks) {
     else
         hipLaunchKernelGGL(k_ts_mark, dim3(kMarkGrid), dim3(kB), 0, st, e.pos_b, e.state_b, e.range, e.d_scenes,
                            t.counts, t.mark_list, t.state_fin);
-    hipLaunchKernelGGL(k_ts_classify, dim3(nblocks(n)), dim3(kB), 0, st, t.state_fin, e.oid_b, n, t.cls);
     e.mark(kStageTwoScaleState);
-    hipLaunchKernelGGL(k_ts_count, dim3(t.nblk), dim3(kB), 0, st, t.cls, n, t.blk, t.nblk);
+    hipLaunchKernelGGL(k_ts_count, dim3(t.nblk), dim3(kB), 0, st, t.state_fin, e.slot_of_oid, n, t.cls, t.blk, t.nblk);
     hipLaunchKernelGGL(k_ts_collect, dim3(t.nblk), dim3(kB), 0, st, t.cls, n, t.blk, t.nblk, t.cap, t.counts,
                        e.status, t.split_ids, t.boundary_ids, t.default_ids);
     e.mark(kStageTwoScaleCollect);
-    hipLaunchKernelGGL(k_ts_seed, dim3(nblocks(t.cap)), dim3(kB), 0, st, t.counts, t.split_ids, t.boundary_ids,
-                       e.slot_of_oid, e.pos_b, e.vel_b, e.d_scenes, t.spos, t.svel, t.sid, t.skey, e.status,
-                       t.sub_cells_valid ? 1 : 0, t.sskey, t.srange);
-    hipLaunchKernelGGL(k_ts_project, dim3(kProjGrid), dim3(kB), 0, st, t.counts, t.spos, t.svel, e.pos_b,
-                       e.vel_b, e.range, e.d_scenes);
+    hipLaunchKernelGGL(k_ts_seed, dim3(kProjGrid + nblocks(t.cap)), dim3(kB), 0, st, t.counts, t.split_ids,
+                       t.boundary_ids, e.slot_of_oid, e.pos_b, e.vel_b, e.range, e.d_scenes, t.spos, t.svel, t.sid,
+                       t.skey, e.status, t.sub_cells_valid ? 1 : 0, t.sskey, t.srange);
     e.mark(kStageTwoScaleSeed);
     sub_pass(e, t, true);
 }
