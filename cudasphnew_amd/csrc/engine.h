@@ -115,6 +115,8 @@ struct Engine {
     // kernel variants of the density / force passes
     sph_tuning tuning = {1, 1, 0, 48, 256};
     uint64_t* masks = nullptr;   // row words [9][N] + chunk masks [3][9][N] (common.h)
+    // the masks pair stands in for the one-lane variants in this plain step
+    bool one_lane_by_masks() const;
 
     // render interop buffers, allocated on the first map
     float4* render_pos = nullptr;   // [N] by original id

@@ -97,6 +97,8 @@ void launch_small_sort(hipStream_t st, const StepBuffers& b, uint32_t cells, con
 // sixteen lanes per particle, the same results bit for bit.  team_step:
 // whether this step's buffers take them, the same answer for both passes.
 bool team_step(const StepBuffers& b);
+// The size rule alone, for sets with and without masks.
+bool team_size(uint32_t n, bool masks);
 void launch_density_team(hipStream_t st, const StepBuffers& b);
 void launch_force_team(hipStream_t st, const StepBuffers& b);
 

@@ -184,7 +184,7 @@ extern "C" sph_status sph_step_noalloc(const sph_params* P, const sph_device_bou
     // and 58 us before, 31 and 30 now at 250,000 particles
     b.masks = reinterpret_cast<uint64_t*>(base + Layout::masks);
     b.plain_masks = true;
-    if (team_step(b)) b.masks = nullptr;
+    if (team_size(n, true)) b.masks = nullptr;
 
     CellSort cs;   // counting sort over the scratch's count array
     cs.cells = (uint32_t)cells;

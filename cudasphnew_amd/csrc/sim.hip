@@ -259,6 +259,21 @@ sph_status Engine::init(int S, const sph_params* P, const sph_scene* scenes) {
         bytes += sorter.bytes();
     }
 
+    // the one-lane variants' masks (one_lane_by_masks): 180 bytes a particle,
+    // unless they are more than an eighth of the free memory; without them
+    // the loops run
+    if (one_lane_by_masks()) {
+        size_t free_bytes = 0, total = 0;
+        const size_t need = sizeof(uint64_t) * row_words_u64(N);
+        if (hipMemGetInfo(&free_bytes, &total) == hipSuccess && need <= free_bytes / 8 &&
+            hipMalloc(&masks, need) == hipSuccess) {
+            bytes += need;
+        } else {
+            (void)hipGetLastError();
+            masks = nullptr;
+        }
+    }
+
     // host staging, then upload
     std::vector<float4> hp(N), hv(N), g4;
     std::vector<uint32_t> ho(N);
@@ -379,6 +394,17 @@ sph_status Engine::resolve_timing() {
     return SPH_OK;
 }
 
+// The one-lane variants of a larger set run as the masks pair with their sums
+// (bit for bit), which saves the force pass its distance tests.  Steps and a
+// position export, loops and masks: two steps of 41,500 particles 187 / 126 us,
+// at twice rest density 291 / 192; four of 400,000 851 / 453.
+// Smaller sets run in teams; batches and two-scale steps (whose split push
+// counts coincident particles) keep the loops.
+bool Engine::one_lane_by_masks() const {
+    return !tuning.hit_masks && tuning.density_lanes == 1 && tuning.force_lanes == 1 && nscenes == 1 &&
+           !team_size(N, true);
+}
+
 void Engine::enqueue_step(bool two_scale) {
     StepBuffers b = buffers();
     mark(kMarkStep);
@@ -403,6 +429,10 @@ void Engine::enqueue_step(bool two_scale) {
     }
     if (!use_cell_sort || !small_sort(N, total_cells)) launch_reorder(stream, b);
     mark(kStageReorder);
+    if (!two_scale && masks && one_lane_by_masks()) {
+        b.masks = masks;
+        b.plain_masks = true;
+    }
     // a two-scale step's split flags come from the hit-mask density pass
     if (two_scale && b.masks) b.split = twoscale_split_refs(*this);
     launch_density(stream, b, tuning.density_lanes, tuning.block);

@@ -329,21 +329,20 @@ void force_team(hipStream_t st, const StepBuffers& b) {
 }
 
 // Teams issue about four times the instructions of one thread per particle,
-// so they win until the chip is full of wavefronts.  Measured over steps of
-// the dam break's block, both passes and the sort, us a step, teams against
-// one thread: 35 / 78 at 4,000 particles, 46 / 78 at 16,384, 64 / 79 at
-// 32,768, 85 / 77 at 50,000 (twice rest density: 132 / 141 there); against
-// the hit-mask pair, two steps and a read of the positions, 118 / 125 at
-// 16,384, 132 / 125 at 20,000 (twice rest density 150 / 187 at 16,384, 204 /
-// 188 at 24,000).  A two-scale step needs the hit-mask density pass's row
-// words and split flags.
-constexpr uint32_t kTeamMax = 40960, kTeamMaxMasks = 18432;
+// so they win until the chip is full of wavefronts.  Against the one-lane
+// loops, us a step with the sort: 35 / 78 at 4,000 particles, 46 / 78 at 16,384,
+// 64 / 79 at 32,768, 85 / 77 at 50,000 (twice rest density: 132 / 141 there);
+// against the masks pair, two steps and a read of the positions: 107 / 119 at
+// 20,000, 117 / 119 at 25,000, 122 / 120 at 30,000 (twice rest density 146 /
+// 187, 160 / 189, 175 / 193).  A two-scale step needs the hit-mask density
+// pass's row words and split flags.
+constexpr uint32_t kTeamMax = 40960, kTeamMaxMasks = 28672;
 
 }  // namespace
 
-bool team_step(const StepBuffers& b) {
-    return b.masks ? b.n <= kTeamMaxMasks && !b.split.state : b.n <= kTeamMax;
-}
+bool team_size(uint32_t n, bool masks) { return n <= (masks ? kTeamMaxMasks : kTeamMax); }
+
+bool team_step(const StepBuffers& b) { return team_size(b.n, b.masks != nullptr) && !b.split.state; }
 
 void launch_density_team(hipStream_t st, const StepBuffers& b) {
     const bool one = b.nscenes == 1;

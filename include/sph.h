@@ -335,7 +335,10 @@ sph_status sph_time_steps(sph_handle* h, int32_t n_steps, int32_t two_scale,
  * the longer rows of a compressed flow) and the force pass runs the pair
  * terms from them through a per-thread hit list of hit_list entries (32, 40,
  * 48 or 64) in LDS, filled as often as a particle's neighbours need;
- * the lanes fields are then unused.  No reference counterpart: the reference
+ * the lanes fields are then unused.  One lane per particle in both passes
+ * (the default) records them too, with the sums of the loops without masks, in
+ * plain steps of one scene of more than 28,672 particles, if the memory is at
+ * most an eighth of what is free.  No reference counterpart: the reference
  * fixes one thread per particle and a block size of 256
  * (particle_simulation.cu:1385-1556, 2943-2957); these generalise its launch
  * configuration. */

@@ -2,7 +2,7 @@
 masks pair stands in for the one-lane kernels (csrc/kernels.hip, PLAIN): bit
 for bit sph_step's default variants.
 
-Sizes at the line (18,432 particles run in teams), a ragged one and the
+Sizes at the line (28,672 particles run in teams), a ragged one and the
 largest; blocks at rest density, 2.2, 4 and 12 times (rows of more than 32 and
 more than 128 candidates), with coincident particles.  A set with a non-finite
 velocity beside a coincident particle leaves its neighbours what the team
@@ -38,7 +38,7 @@ def hip_stream():
     hip.hipStreamDestroy(stream)
 
 
-@pytest.mark.parametrize("n,crowd,steps", [(18432, 1.0, 1), (18433, 1.0, 2), (45001, 2.2, 2), (45000, 12.0, 2),
+@pytest.mark.parametrize("n,crowd,steps", [(28672, 1.0, 1), (28673, 1.0, 2), (45001, 2.2, 2), (45000, 12.0, 2),
                                            (100003, 1.0, 1), (262144, 4.0, 3)])
 def test_large_set_equals_handle(hip_stream, n, crowd, steps):
     hip, stream = hip_stream
