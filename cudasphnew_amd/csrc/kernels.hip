@@ -245,11 +245,34 @@ __global__ __launch_bounds__(kBlock) void k_density_coop(const float4* __restric
     reinterpret_cast<float*>(vel)[4 * (size_t)s + 3] = rho;
 }
 
+// The pair terms of a run [b, e) of candidates, in order.  Per 64 of them a
+// cheap distance test records the hits in a 64-bit mask, then the pair terms
+// run for the set bits only: roughly one candidate in six is within h, so a
+// fused loop would run the pair body for almost every candidate of a wavefront.
+__device__ __forceinline__ void scan_run(PairSums& a, const float4* __restrict__ pos, const float4* __restrict__ vel,
+                                         int b, int e, float4 xi, float4 vi, float Ai, const DevScene& S, float kr0) {
+    const float h = S.h, h2 = S.h2;
+    for (int base = b; base < e; base += 64) {
+        const int cnt = min(64, e - base);
+        uint64_t hits = 0;
+#pragma unroll 4
+        for (int t = 0; t < cnt; ++t) {
+            float4 xj = pos[base + t];
+            float dx = xi.x - xj.x, dy = xi.y - xj.y, dz = xi.z - xj.z;
+            float r2 = sq3(dx, dy, dz);
+            hits |= (uint64_t)(r2 <= h2 && r2 > 0.0f) << t;
+        }
+        while (hits) {
+            const int t = __ffsll((unsigned long long)hits) - 1;
+            hits &= hits - 1;
+            const int q = base + t;
+            pair_terms(a, xi, vi, vi.w, Ai, h, h2, S.stiff, kr0, pos[q], vel[q]);
+        }
+    }
+}
+
 // compute_particle_acceleration_ifsurf (cu:315-474, 1459-1556) + integration,
-// one thread per particle.  Per run of up to 64 candidates a cheap distance
-// test records the hits in a 64-bit mask, then the pair terms run for the
-// set bits only: roughly one candidate in six is within h, so a fused loop
-// would run the pair body for almost every candidate of a wavefront.
+// one thread per particle.
 template <int B, bool ONE>
 __global__ __launch_bounds__(B) void k_force(
     const float4* __restrict__ pos, const float4* __restrict__ vel, const int2* __restrict__ range, uint32_t n,
@@ -264,7 +287,6 @@ __global__ __launch_bounds__(B) void k_force(
     const float4 xi = pos[s];
     const float4 vi = vel[s];
     const float rhoi = vi.w;
-    const float h = S.h, h2 = S.h2;
     const float Ai = S.stiff * (rhoi - S.rho0) / rhoi;   // p_i / rho_i
     const float kr0 = S.stiff * S.rho0;
     Rows R = neighbour_rows(S, xi);
@@ -273,23 +295,7 @@ __global__ __launch_bounds__(B) void k_force(
         for (int dj = 0; dj < 3; ++dj) {
             int b, e;
             row_slots(range, S, R, dk, dj, xi, b, e);
-            for (int base = b; base < e; base += 64) {
-                const int cnt = min(64, e - base);
-                uint64_t hits = 0;
-#pragma unroll 4
-                for (int t = 0; t < cnt; ++t) {
-                    float4 xj = pos[base + t];
-                    float dx = xi.x - xj.x, dy = xi.y - xj.y, dz = xi.z - xj.z;
-                    float r2 = sq3(dx, dy, dz);
-                    hits |= (uint64_t)(r2 <= h2 && r2 > 0.0f) << t;
-                }
-                while (hits) {
-                    const int t = __ffsll((unsigned long long)hits) - 1;
-                    hits &= hits - 1;
-                    const int q = base + t;
-                    pair_terms(a, xi, vi, rhoi, Ai, h, h2, S.stiff, kr0, pos[q], vel[q]);
-                }
-            }
+            scan_run(a, pos, vel, b, e, xi, vi, Ai, S, kr0);
         }
     force_finish(S, s, xi, vi, a, grid4, gridd, oid_b, state_b, acc, pos_out, vel_out, oid_out, state_out, key_out,
                  status, nr, by_id);
@@ -606,7 +612,8 @@ __device__ __forceinline__ bool wave_span(uint32_t b, int e, uint32_t& lo, int& 
 constexpr int kWin = 192;
 
 // PLAIN: the arithmetic of k_density, bit for bit (the pair of masks kernels
-// in place of the one-lane kernels).
+// in place of the one-lane kernels), and its loop where no lane's row wants
+// bits: 120,000 particles at ten times rest density 157 -> 147 us, k_density 147.
 template <int B, bool ONE, bool PLAIN = false>
 __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_density_masks(const float4* __restrict__ pos, float4* __restrict__ vel,
                                                      const int2* __restrict__ range, uint32_t n,
@@ -667,6 +674,13 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(8, 8))) void 
                 // a lane without a run reads nothing; its place is any
                 m = density_row<PLAIN>(WindowRow{win + __umul24(b - lo, 3)}, cnt, xi, h2, self, sum, put);
                 wave_sync();   // the next row's window replaces this one
+            } else if (PLAIN && __all(cnt == 0 || cnt > kRowMaxCands)) {
+                // no bits wanted: k_density's loop
+#pragma unroll 4
+                for (int q = (int)b; q < (int)b + cnt; ++q) {
+                    const float d = density_gap(xi, pos[q], h2);
+                    sum += d * d * d;
+                }
             } else if (some) {
                 m = density_row<PLAIN>(GlobalRow{pb, b}, cnt, xi, h2, self, sum, put);
             }
@@ -728,8 +742,13 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(8, 8))) void 
 // spills and takes 139 us (156 us with two gathers in flight instead of
 // three).
 //
-// PLAIN: the sums of k_force, bit for bit: a particle with a row past
-// kRowMaxCands scans all its rows in order.
+// PLAIN: the sums of k_force, bit for bit.  A wavefront with a row past
+// kRowMaxCands takes all its rows in order, without the list: a row's hits
+// come from its words, those of a long one from k_force's scan.  35,000 and
+// 120,000 particles at four times rest density: 117 and 135 us (k_force 150 and
+// 177), 250 and 259 with the candidates of all rows tested and evaluated one by
+// one in the lanes with a long row; 120,000 at ten times, nearly every row
+// long: 395, k_force 389, one by one 509.
 template <int CAP, int B, bool ONE, bool PLAIN = false>
 __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(CAP <= 40 ? 5 : (CAP <= 48 ? 4 : 3), 8))) void k_force_masks(
     const float4* __restrict__ pos, const float4* __restrict__ vel, const int2* __restrict__ range, uint32_t n,
@@ -766,12 +785,7 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(CAP <= 40 ? 5
                 s_base[row][tid] = (int)row_first(mk[row]);
             }
         }
-        if (PLAIN && long_rows) {
-            long_rows = 0x1FFu;
-            last = 0u;
-#pragma unroll
-            for (int row = 0; row < 9; ++row) bits[row] = 0u;
-        }
+        const bool in_order = PLAIN && __any(long_rows != 0u);
         const uint32_t* const cm = chunk_masks(masks, n);
         const float4 xi = pos[s];
         const float4 vi = vel[s];
@@ -781,8 +795,33 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(CAP <= 40 ? 5
         const float kr0 = S.stiff * S.rho0;
         PairSums a = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
         const F4Buf pb(pos), vb(vel);
+        if (in_order) {
+            const Rows R = neighbour_rows(S, xi);
+    #pragma unroll 1
+            for (int row = 0; row < 9; ++row) {
+                const uint64_t w = masks[(size_t)row * n + s];
+                if (w == kRowLong) {
+                    int b, e;
+                    row_slots(range, S, R, row / 3, row % 3, xi, b, e);
+                    scan_run(a, pos, vel, b, e, xi, vi, Ai, S, kr0);
+                    continue;
+                }
+                const uint32_t lc = row_last_chunk(w);
+                // two chunks at a time
+                for (uint32_t c = 0; c <= lc; c += 2) {
+                    const uint32_t q0 = row_first(w) + 32u * c;
+                    uint64_t hits = c == 0 ? (uint32_t)w : cm[chunk_at(n, c, row, s)];
+                    if (c < lc) hits |= (uint64_t)cm[chunk_at(n, c + 1, row, s)] << 32;
+                    while (hits) {
+                        const uint32_t q = q0 + (uint32_t)__builtin_ctzll(hits);
+                        hits &= hits - 1;
+                        pair_terms(a, xi, vi, rhoi, Ai, h, h2, S.stiff, kr0, pb[q], vb[q]);
+                    }
+                }
+            }
+        }
         int m;
-        do {
+        if (!in_order) do {
             m = 0;
     #pragma unroll
             for (int row = 0; row < 9; ++row) {
@@ -839,7 +878,7 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(CAP <= 40 ? 5
                 if (k + 2 < m) pair_terms<!PLAIN>(a, xi, vi, rhoi, Ai, h, h2, S.stiff, kr0, x2, v2);
             }
         } while (m == CAP);   // a full list: hits may remain
-        if (long_rows) {
+        if (!PLAIN && long_rows) {
             // rows of more than kRowMaxCands candidates: scanned here
             const Rows R = neighbour_rows(S, xi);
     #pragma unroll 1
