@@ -13,6 +13,7 @@
 #include "cell_sort.h"
 #include "host_copy.h"
 #include "kernels.h"
+#include "on_device.h"
 #include "radix_sort.h"
 
 namespace sph {

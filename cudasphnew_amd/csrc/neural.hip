@@ -1097,6 +1097,7 @@ struct sph_mlp {
     float* eval_buf = nullptr;   // sph_mlp_eval: points, then results
     size_t eval_bytes = 0;
     sph::HostCopy reader;
+    int device = 0;
     hipStream_t stream = nullptr;
     std::string err;
 
@@ -1192,6 +1193,7 @@ sph_status neural_attach(Engine& e, int scene, sph_mlp* m, const float* val, siz
     if (!m || (nval && !val)) return e.fail(SPH_INVALID_ARG, "network required");
     if (!(cfg.tolerance > 0.0f) || !(cfg.band > 0.0f) || cfg.brick < 1)
         return e.fail(SPH_INVALID_ARG, "tolerance and band must be positive and brick >= 1");
+    const OnDevice current(e.device);
     if (!e.nb) {
         NeuralBoundary* nb = new (std::nothrow) NeuralBoundary();
         if (!nb) return SPH_OUT_OF_MEMORY;
@@ -1368,6 +1370,7 @@ sph_status sph_mlp_create(const sph_mlp_config* cfg, sph_mlp** out) {
     sph_mlp* h = new (std::nothrow) sph_mlp();
     if (!h) return SPH_OUT_OF_MEMORY;
     h->cfg = *cfg;
+    h->device = dev;
     int cus = 256;
     (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
     h->nblocks = cus;   // one partial gradient vector per CU
@@ -1450,6 +1453,7 @@ sph_status sph_mlp_get_params(sph_mlp* h, float* params, size_t n) {
 
 sph_status sph_mlp_set_samples(sph_mlp* h, const float* xyzd, size_t n) {
     if (!h || !xyzd || n < (size_t)kTile || n > 0xFFFFFFFFull) return h ? h->fail(SPH_INVALID_ARG, "need >= 64 samples") : SPH_INVALID_ARG;
+    const sph::OnDevice on(h->device);
     if (h->samples) (void)hipFree(h->samples);
     h->samples = nullptr;
     if (hipMalloc(&h->samples, sizeof(float4) * n) != hipSuccess) {
@@ -1493,6 +1497,7 @@ sph_status sph_mlp_gradient(sph_mlp* h, uint32_t first, int32_t batch, float* gr
     if (!h || !grad || !loss) return SPH_INVALID_ARG;
     if (!h->samples) return h->fail(SPH_INVALID_ARG, "no samples");
     if (batch < kTile || batch % kTile) return h->fail(SPH_INVALID_ARG, "batch must be a positive multiple of 64");
+    const sph::OnDevice on(h->device);
     float* dloss = nullptr;
     if (hipMalloc(&dloss, sizeof(float)) != hipSuccess) return h->fail(SPH_OUT_OF_MEMORY, "alloc");
     sph_status st = enqueue_pass(h, first % h->nsamples, batch, false, h->grad, dloss);
@@ -1510,6 +1515,7 @@ sph_status sph_mlp_train(sph_mlp* h, int32_t steps, int32_t batch, float* losses
     if (!h || steps < 0) return SPH_INVALID_ARG;
     if (!h->samples) return h->fail(SPH_INVALID_ARG, "no samples");
     if (batch < kTile || batch % kTile) return h->fail(SPH_INVALID_ARG, "batch must be a positive multiple of 64");
+    const sph::OnDevice on(h->device);
     if (steps > h->loss_cap) {
         if (h->loss) (void)hipFree(h->loss);
         h->loss = nullptr;
@@ -1539,6 +1545,7 @@ sph_status sph_mlp_eval(sph_mlp* h, const float* xyz, size_t n, float* dgrad) {
     if (!h || (n && (!xyz || !dgrad))) return SPH_INVALID_ARG;
     if (n == 0) return SPH_OK;
     if (n > 0xFFFFFFFFull) return h->fail(SPH_INVALID_ARG, "too many points");
+    const sph::OnDevice on(h->device);
     // points and results in one buffer, kept with the handle up to
     // kEvalKeep bytes; larger ones are given back after the call
     const size_t out_at = (3 * n + 3) / 4 * 4, bytes = sizeof(float) * (out_at + 4 * n);
@@ -1580,6 +1587,7 @@ sph_status sph_mlp_get_config(const sph_mlp* h, sph_mlp_config* out) {
 
 sph_status sph_mlp_time_train(sph_mlp* h, int32_t steps, int32_t batch, float* ms) {
     if (!h || !ms || steps < 1) return SPH_INVALID_ARG;
+    const sph::OnDevice on(h->device);
     hipEvent_t a, b;
     if (hipEventCreate(&a) != hipSuccess || hipEventCreate(&b) != hipSuccess) return SPH_DEVICE_ERROR;
     (void)hipEventRecord(a, h->stream);

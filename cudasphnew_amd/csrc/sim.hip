@@ -127,6 +127,7 @@ sph_status Engine::fail(sph_status s, const std::string& msg) {
 
 template <class T>
 sph_status Engine::alloc(T** p, size_t count) {
+    const OnDevice on(device);
     size_t b = sizeof(T) * (count ? count : 1);
     hipError_t e = hipMalloc(reinterpret_cast<void**>(p), b);
     if (e != hipSuccess) {
@@ -358,6 +359,7 @@ StepBuffers Engine::buffers() const {
 
 hipEvent_t Engine::next_event() {
     if (ev_used == ev_pool.size()) {
+        const OnDevice on(device);
         hipEvent_t e = nullptr;
         if (hipEventCreate(&e) != hipSuccess) return nullptr;
         ev_pool.push_back(e);
@@ -455,6 +457,7 @@ void Engine::enqueue_step(bool two_scale) {
 sph_status Engine::step(int n, bool two_scale) {
     if (n < 0) return fail(SPH_INVALID_ARG, "n_steps must be >= 0");
     if (two_scale && !ts) {
+        const OnDevice on(device);
         sph_status st = twoscale_create(*this);
         if (st != SPH_OK) return st;
         drop_graph();   // the step's buffers now include the sub-particle pass's
@@ -599,6 +602,7 @@ sph_status Engine::alias_distance() {
 
 sph_status Engine::own_distance() {
     if (!gridd_alias) return SPH_OK;
+    const OnDevice on(device);
     float* p = nullptr;
     const size_t nb = sizeof(float) * (grid_nodes ? grid_nodes : 1);
     if (hipMalloc(&p, nb) != hipSuccess) {
@@ -675,6 +679,7 @@ sph_status Engine::autotune(int reps, sph_tuning* out) {
     if (last_two_scale && ts) plain.state_b = twoscale_final_state(*this);
     StepBuffers withm = plain;
     withm.masks = masks;
+    const OnDevice on(device);
     hipEvent_t e0 = nullptr, e1 = nullptr;
     if (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess) {
         if (e0) (void)hipEventDestroy(e0);
@@ -758,6 +763,7 @@ sph_status Engine::autotune(int reps, sph_tuning* out) {
 // 100,000, 72 -> 39 at 16,384.
 sph_status Engine::read_floats(int s, sph_field f, float* dst, size_t nbytes) {
     const uint32_t b = hbegins[s], n = hbegins[s + 1] - b;
+    const OnDevice on(device);   // the pinned slots and events
     if (!read_stage) {
         uint32_t most = 0;
         for (int k = 0; k < nscenes; ++k) most = std::max(most, hbegins[k + 1] - hbegins[k]);
@@ -1145,6 +1151,7 @@ const char* sph_stage_name(int32_t stage) { return sph::stage_name(stage); }
 
 static sph_status time_engine(Engine& e, int32_t n, bool two_scale, float* ms) {
     if (!ms || n < 1) return SPH_INVALID_ARG;
+    const sph::OnDevice on(e.device);
     hipEvent_t a, b;
     if (hipEventCreate(&a) != hipSuccess || hipEventCreate(&b) != hipSuccess) return SPH_DEVICE_ERROR;
     (void)hipEventRecord(a, e.stream);
