@@ -19,7 +19,7 @@ namespace sph {
 struct HostCopy {
     static constexpr size_t kChunk = 512u << 10;
     static constexpr int kSlots = 4;
-    static constexpr size_t kTail = 64;   // a small extra record (a status word) behind the slots
+    static constexpr size_t kTail = 64;   // the status word, behind the slots
 
     char* pin = nullptr;
     hipEvent_t done[kSlots] = {};
@@ -48,14 +48,14 @@ struct HostCopy {
     }
 
     // bytes of device memory src into dst, after the work on st; waits for
-    // them.  extra (at most kTail bytes, may be null): a device record read at
-    // the same time, valid in tail() afterwards.
-    hipError_t read(hipStream_t st, void* dst, const void* src, size_t bytes, const void* extra = nullptr,
-                    size_t extra_bytes = 0) {
+    // them.  word (may be null): a device status word, copied first; nothing
+    // is written to dst unless accept takes its value.
+    template <class Accept>
+    hipError_t read(hipStream_t st, void* dst, const void* src, size_t bytes, const uint32_t* word, Accept accept) {
         hipError_t e = init();
         if (e != hipSuccess) return e;
-        if (extra) {
-            e = hipMemcpyAsync(tail(), extra, extra_bytes, hipMemcpyDeviceToHost, st);
+        if (word) {
+            e = hipMemcpyAsync(pinned_word(), word, sizeof(uint32_t), hipMemcpyDeviceToHost, st);
             if (e != hipSuccess) return e;
         }
         const size_t n = (bytes + kChunk - 1) / kChunk;
@@ -70,6 +70,7 @@ struct HostCopy {
         for (size_t k = 0; k < n && e == hipSuccess; ++k) {
             if (n > 1) e = hipEventSynchronize(done[k % kSlots]);
             if (e != hipSuccess) break;
+            if (k == 0 && word && !accept(*pinned_word())) return hipStreamSynchronize(st);
             std::memcpy(static_cast<char*>(dst) + k * kChunk, pin + k % kSlots * kChunk, size(k));
             if (k + kSlots < n) e = send(k + kSlots);
         }
@@ -77,7 +78,12 @@ struct HostCopy {
         return e;
     }
 
-    void* tail() const { return pin + kChunk * kSlots; }
+    hipError_t read(hipStream_t st, void* dst, const void* src, size_t bytes) {
+        return read(st, dst, src, bytes, nullptr, [](uint32_t) { return true; });
+    }
+
+  private:
+    uint32_t* pinned_word() const { return reinterpret_cast<uint32_t*>(pin + kChunk * kSlots); }
 };
 
 }  // namespace sph

@@ -778,12 +778,14 @@ sph_status Engine::read_floats(int s, sph_field f, float* dst, size_t nbytes) {
                         oid_a + b, read_stage);
     sph_status st = check_launch("field read");
     if (st != SPH_OK) return st;
-    if (reader.read(stream, dst, read_stage, nbytes, status, sizeof(uint32_t)) != hipSuccess)
+    auto accept = [&](uint32_t word) {
+        st = status_of(word);
+        if (st == SPH_OUT_OF_DOMAIN || st == SPH_NONFINITE_STATE) st = SPH_OK;
+        return st == SPH_OK;
+    };
+    if (reader.read(stream, dst, read_stage, nbytes, status, accept) != hipSuccess)
         return fail(SPH_DEVICE_ERROR, "device-to-host copy failed");
-    uint32_t word;
-    std::memcpy(&word, reader.tail(), sizeof(word));
-    st = status_of(word);
-    return st == SPH_OUT_OF_DOMAIN || st == SPH_NONFINITE_STATE ? SPH_OK : st;
+    return st;
 }
 
 sph_status Engine::read_field(int s, sph_field f, void* dst, size_t nbytes) {
