@@ -14,28 +14,33 @@ namespace sph {
 // KiB, 220 for 384 KiB, 1000 for 4 MiB, 2910 for 12 MiB.  Through pinned slots
 // (a chunk crosses the bus while the host copies the one before it) 19, 71,
 // 750 and 2220 us; up to a chunk there is nothing to overlap and one copy is
-// the fastest.  Each owner has its own slots, allocated on first use and freed
-// with it.
+// the fastest.  Each owner has its own slots, allocated on first use -- one
+// for reads of up to a chunk, all with the first larger one -- and freed with
+// it.
 struct HostCopy {
     static constexpr size_t kChunk = 512u << 10;
     static constexpr int kSlots = 4;
     static constexpr size_t kTail = 64;   // the status word, behind the slots
 
     char* pin = nullptr;
+    int slots = 0;
     hipEvent_t done[kSlots] = {};
 
     HostCopy() = default;
     HostCopy(const HostCopy&) = delete;
     HostCopy& operator=(const HostCopy&) = delete;
 
-    hipError_t init() {
-        if (pin) return hipSuccess;
-        for (int i = 0; i < kSlots; ++i) {
-            if (done[i]) continue;
+    hipError_t init(size_t bytes) {
+        const int want = bytes <= kChunk ? 1 : kSlots;
+        if (slots >= want) return hipSuccess;
+        release();
+        for (int i = 0; i < want && want > 1; ++i) {
             hipError_t e = hipEventCreateWithFlags(&done[i], hipEventDisableTiming);
             if (e != hipSuccess) return e;
         }
-        return hipHostMalloc(reinterpret_cast<void**>(&pin), kChunk * kSlots + kTail, 0);
+        hipError_t e = hipHostMalloc(reinterpret_cast<void**>(&pin), kChunk * want + kTail, 0);
+        if (e == hipSuccess) slots = want;
+        return e;
     }
 
     void release() {
@@ -45,6 +50,7 @@ struct HostCopy {
             e = nullptr;
         }
         pin = nullptr;
+        slots = 0;
     }
 
     // bytes of device memory src into dst, after the work on st; waits for
@@ -52,7 +58,7 @@ struct HostCopy {
     // is written to dst unless accept takes its value.
     template <class Accept>
     hipError_t read(hipStream_t st, void* dst, const void* src, size_t bytes, const uint32_t* word, Accept accept) {
-        hipError_t e = init();
+        hipError_t e = init(bytes);
         if (e != hipSuccess) return e;
         if (word) {
             e = hipMemcpyAsync(pinned_word(), word, sizeof(uint32_t), hipMemcpyDeviceToHost, st);
@@ -83,7 +89,7 @@ struct HostCopy {
     }
 
   private:
-    uint32_t* pinned_word() const { return reinterpret_cast<uint32_t*>(pin + kChunk * kSlots); }
+    uint32_t* pinned_word() const { return reinterpret_cast<uint32_t*>(pin + kChunk * slots); }
 };
 
 }  // namespace sph
