@@ -147,6 +147,7 @@ struct Engine {
     sph_status alloc(T** p, size_t count);
     sph_status status_of(uint32_t word);   // error of a device status word
     sph_status read_floats(int scene, sph_field f, float* dst, size_t nbytes);
+    sph_status read_floats_by_host(int scene, sph_field f, float* dst);
     sph_status read_field(int scene, sph_field f, void* dst, size_t bytes_out);
     sph_status upload_params(int scene, const sph_params& p);
     sph_status map_render(sph_render_view* out);

@@ -16,7 +16,7 @@ namespace sph {
 // 750 and 2220 us; up to a chunk there is nothing to overlap and one copy is
 // the fastest.  Each owner has its own slots, allocated on first use -- one
 // for reads of up to a chunk, all with the first larger one -- and freed with
-// it.
+// it.  Where they cannot be had the runtime's own path serves.
 struct HostCopy {
     static constexpr size_t kChunk = 512u << 10;
     static constexpr int kSlots = 4;
@@ -58,8 +58,11 @@ struct HostCopy {
     // is written to dst unless accept takes its value.
     template <class Accept>
     hipError_t read(hipStream_t st, void* dst, const void* src, size_t bytes, const uint32_t* word, Accept accept) {
-        hipError_t e = init(bytes);
-        if (e != hipSuccess) return e;
+        if (init(bytes) != hipSuccess) {
+            (void)hipGetLastError();
+            return read_direct(st, dst, src, bytes, word, accept);
+        }
+        hipError_t e = hipSuccess;
         if (word) {
             e = hipMemcpyAsync(pinned_word(), word, sizeof(uint32_t), hipMemcpyDeviceToHost, st);
             if (e != hipSuccess) return e;
@@ -89,6 +92,22 @@ struct HostCopy {
     }
 
   private:
+    template <class Accept>
+    static hipError_t read_direct(hipStream_t st, void* dst, const void* src, size_t bytes, const uint32_t* word,
+                                  Accept accept) {
+        uint32_t value = 0;
+        hipError_t e = hipSuccess;
+        if (word) {
+            e = hipMemcpyAsync(&value, word, sizeof(value), hipMemcpyDeviceToHost, st);
+            const hipError_t w = hipStreamSynchronize(st);
+            if (e == hipSuccess) e = w;
+            if (e != hipSuccess || !accept(value)) return e;
+        }
+        e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, st);
+        const hipError_t w = hipStreamSynchronize(st);
+        return e == hipSuccess ? w : e;
+    }
+
     uint32_t* pinned_word() const { return reinterpret_cast<uint32_t*>(pin + kChunk * slots); }
 };
 

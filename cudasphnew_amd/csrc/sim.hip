@@ -767,8 +767,14 @@ sph_status Engine::read_floats(int s, sph_field f, float* dst, size_t nbytes) {
     if (!read_stage) {
         uint32_t most = 0;
         for (int k = 0; k < nscenes; ++k) most = std::max(most, hbegins[k + 1] - hbegins[k]);
-        sph_status st = alloc(&read_stage, 3 * (size_t)most);
-        if (st != SPH_OK) return st;
+        const size_t need = 3 * sizeof(float) * (size_t)most;
+        if (hipMalloc(reinterpret_cast<void**>(&read_stage), need) == hipSuccess) {
+            bytes += need;
+        } else {
+            (void)hipGetLastError();
+            read_stage = nullptr;
+            return read_floats_by_host(s, f, dst);
+        }
     }
     if (f == SPH_FIELD_DENSITY || f == SPH_FIELD_PRESSURE)
         launch_read_density(stream, n, vel_a + b, oid_a + b, f == SPH_FIELD_PRESSURE, params[s].gas_stiffness,
@@ -786,6 +792,28 @@ sph_status Engine::read_floats(int s, sph_field f, float* dst, size_t nbytes) {
     if (reader.read(stream, dst, read_stage, nbytes, status, accept) != hipSuccess)
         return fail(SPH_DEVICE_ERROR, "device-to-host copy failed");
     return st;
+}
+
+// The same without memory for the scattered field: the records and ids as they
+// are stored, scattered by the host.
+sph_status Engine::read_floats_by_host(int s, sph_field f, float* dst) {
+    sph_status st = sync();
+    if (st != SPH_OK && st != SPH_OUT_OF_DOMAIN && st != SPH_NONFINITE_STATE) return st;
+    const uint32_t b = hbegins[s], n = hbegins[s + 1] - b;
+    const float4* src = f == SPH_FIELD_POSITION ? pos_a : (f == SPH_FIELD_ACCEL ? acc : vel_a);
+    std::vector<float4> rec(n);
+    std::vector<uint32_t> oid(n);
+    if (hipMemcpy(rec.data(), src + b, n * sizeof(float4), hipMemcpyDeviceToHost) != hipSuccess ||
+        hipMemcpy(oid.data(), oid_a + b, n * sizeof(uint32_t), hipMemcpyDeviceToHost) != hipSuccess)
+        return fail(SPH_DEVICE_ERROR, "device-to-host copy failed");
+    const sph_params& P = params[s];
+    for (uint32_t i = 0; i < n; ++i) {
+        const float4 r = rec[i];
+        if (f == SPH_FIELD_DENSITY) dst[oid[i]] = r.w;
+        else if (f == SPH_FIELD_PRESSURE) dst[oid[i]] = P.gas_stiffness * (r.w - P.rest_density);
+        else std::memcpy(dst + 3 * (size_t)oid[i], &r, 3 * sizeof(float));
+    }
+    return SPH_OK;
 }
 
 sph_status Engine::read_field(int s, sph_field f, void* dst, size_t nbytes) {
