@@ -219,19 +219,23 @@ def cpu_baseline(scene, seconds: float, threads: int):
     }
 
 
-def kernel_name(stage: str, tuning: dict, one_scene: bool = True) -> str:
-    """The kernel (as rocprofv3 names it, template arguments included) that a
-    stage launched under the given variants."""
+def kernel_name(stage: str, tuning: dict, n: int, one_scene: bool = True) -> str:
+    """The kernel (as the profile summaries name it, template arguments
+    included) that a stage of a plain step of n particles launches under the
+    given variants."""
     b, one = tuning["block"], "true" if one_scene else "false"
-    if stage == "force":
-        if tuning["hit_masks"]:
-            return f"k_force_masks<{tuning['hit_list']},{b},{one}>"
-        return f"k_force<{b},{one}>" if tuning["force_lanes"] == 1 else f"k_force_coop<{tuning['force_lanes']}>"
-    if stage == "density":
-        if tuning["hit_masks"]:
-            return f"k_density_masks<{b},{one}>"
-        return f"k_density<{b},{one}>" if tuning["density_lanes"] == 1 else \
-            f"k_density_coop<{tuning['density_lanes']}>"
+    masks, lanes = bool(tuning["hit_masks"]), (tuning["density_lanes"], tuning["force_lanes"])
+    if stage in ("density", "force"):
+        own = lanes[stage == "force"]
+        # one lane in both passes of a larger scene runs as the masks pair
+        plain = one_scene and not masks and lanes == (1, 1) and n > 28672
+        # small sets run in teams of sixteen lanes (csrc/team.hip)
+        if (masks or own == 1) and not plain and n <= (28672 if masks else 40960):
+            return f"k_{stage}_team<{'true' if masks else 'false'},{one}>"
+        if masks or plain:
+            cap = f"{48 if plain else tuning['hit_list']}," if stage == "force" else ""
+            return f"k_{stage}_masks<{cap}{256 if plain else b},{one}{',plain' if plain else ''}>"
+        return f"k_{stage}<{b},{one}>" if own == 1 else f"k_{stage}_coop<{own}>"
     if stage == "reorder":
         return f"k_reorder<{'false' if one_scene else 'true'}>"
     return f"k_{stage}"
@@ -580,7 +584,7 @@ def main(argv=None) -> int:
     algo_bytes = algo[dom]
     t_dom = single[dom] / 1e3
     achieved = algo_bytes / t_dom / 1e9
-    kname = kernel_name(dom, tuning)
+    kname = kernel_name(dom, tuning, n)
     roofline = {
         "bound": "hbm",
         "kernel": kname,
@@ -600,11 +604,11 @@ def main(argv=None) -> int:
         "touched_cells": tc,
         "touched_texels": tex,
         # every neighbour pass and streaming pass of the step on the same footing
-        "stages": {k: {"kernel": kernel_name(k, tuning), "avg_launch_ms": round(single[k], 5),
+        "stages": {k: {"kernel": kernel_name(k, tuning, n), "avg_launch_ms": round(single[k], 5),
                        "algorithmic_bytes": int(algo[k]),
                        "frac": round(algo[k] / (single[k] / 1e3) / 1e9 / HBM_PEAK_GBS, 5),
-                       "traffic": profiled_traffic(a.config, kernel_name(k, tuning)),
-                       "profiled_busy": profiled_busy(a.config, kernel_name(k, tuning))}
+                       "traffic": profiled_traffic(a.config, kernel_name(k, tuning, n)),
+                       "profiled_busy": profiled_busy(a.config, kernel_name(k, tuning, n))}
                    for k in single},
     }
     forms = None

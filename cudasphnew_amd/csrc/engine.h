@@ -116,8 +116,10 @@ struct Engine {
     // kernel variants of the density / force passes
     sph_tuning tuning = {1, 1, 0, 48, 256};
     uint64_t* masks = nullptr;   // row words [9][N] + chunk masks [3][9][N] (common.h)
-    // the masks pair stands in for the one-lane variants in this plain step
-    bool one_lane_by_masks() const;
+    // the masks pair stands in for the one-lane variants t in such a step
+    bool one_lane_by_masks(const sph_tuning& t, bool two_scale) const;
+    // sets what selects the two passes' kernels under variants t
+    void route(StepBuffers& b, const sph_tuning& t, bool two_scale) const;
 
     // render interop buffers, allocated on the first map
     float4* render_pos = nullptr;   // [N] by original id

@@ -43,6 +43,8 @@ struct StepBuffers {
     uint64_t* masks = nullptr;
     // masks with the one-lane variants' results bit for bit (one scene)
     bool plain_masks = false;
+    // the team kernels may stand in for the one-lane and hit-mask variants
+    bool teams = true;
     // the force pass's positions and velocities go to pos_a[id], vel_a[id]
     // instead of storage order (the one-lane, team and masks variants; the last
     // step of a call that returns its particles by id)

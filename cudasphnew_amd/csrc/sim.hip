@@ -263,7 +263,7 @@ sph_status Engine::init(int S, const sph_params* P, const sph_scene* scenes) {
     // the one-lane variants' masks (one_lane_by_masks): 180 bytes a particle,
     // unless they are more than an eighth of the free memory; without them
     // the loops run
-    if (one_lane_by_masks()) {
+    if (one_lane_by_masks(tuning, false)) {
         size_t free_bytes = 0, total = 0;
         const size_t need = sizeof(uint64_t) * row_words_u64(N);
         if (hipMemGetInfo(&free_bytes, &total) == hipSuccess && need <= free_bytes / 8 &&
@@ -347,7 +347,6 @@ StepBuffers Engine::buffers() const {
     b.slot_of_oid = ts ? slot_of_oid : nullptr;
     b.range = range;
     b.status = status;
-    b.masks = tuning.hit_masks ? masks : nullptr;
     b.nr.mode = wall_mode;
     b.nr.skey = skey;
     b.nr.rec = neural_records(*this);
@@ -402,9 +401,25 @@ sph_status Engine::resolve_timing() {
 // at twice rest density 291 / 192; four of 400,000 851 / 453.
 // Smaller sets run in teams; batches and two-scale steps (whose split push
 // counts coincident particles) keep the loops.
-bool Engine::one_lane_by_masks() const {
-    return !tuning.hit_masks && tuning.density_lanes == 1 && tuning.force_lanes == 1 && nscenes == 1 &&
+bool Engine::one_lane_by_masks(const sph_tuning& t, bool two_scale) const {
+    return !two_scale && !t.hit_masks && t.density_lanes == 1 && t.force_lanes == 1 && nscenes == 1 &&
            !team_size(N, true);
+}
+
+// The kernels of a step's density and force passes under variants t; the
+// autotuner times what this selects.
+void Engine::route(StepBuffers& b, const sph_tuning& t, bool two_scale) const {
+    const bool plain = one_lane_by_masks(t, two_scale);
+    b.masks = t.hit_masks || plain ? masks : nullptr;
+    b.plain_masks = plain && masks;
+    // the masks pair of a two-scale step: its density pass pushes the split
+    // flags, its row words serve the marking pass
+    b.teams = !(two_scale && t.hit_masks);
+}
+
+static void launch_passes(hipStream_t st, const StepBuffers& b, const sph_tuning& t, bool density, bool force) {
+    if (density) launch_density(st, b, t.density_lanes, t.block);
+    if (force) launch_force(st, b, t.hit_masks ? t.hit_list : t.force_lanes, t.block);
 }
 
 void Engine::enqueue_step(bool two_scale) {
@@ -431,13 +446,10 @@ void Engine::enqueue_step(bool two_scale) {
     }
     if (!use_cell_sort || !small_sort(N, total_cells)) launch_reorder(stream, b);
     mark(kStageReorder);
-    if (!two_scale && masks && one_lane_by_masks()) {
-        b.masks = masks;
-        b.plain_masks = true;
-    }
+    route(b, tuning, two_scale);
     // a two-scale step's split flags come from the hit-mask density pass
     if (two_scale && b.masks) b.split = twoscale_split_refs(*this);
-    launch_density(stream, b, tuning.density_lanes, tuning.block);
+    launch_passes(stream, b, tuning, true, false);
     mark(kStageDensity);
     if (two_scale) {
         twoscale_enqueue(*this, b.masks);
@@ -447,7 +459,7 @@ void Engine::enqueue_step(bool two_scale) {
         neural_enqueue(*this);   // normals where the density pass found the wall penalty active
         mark(kStageWallMlp);
     }
-    launch_force(stream, b, tuning.hit_masks ? tuning.hit_list : tuning.force_lanes, tuning.block);
+    launch_passes(stream, b, tuning, false, true);
     mark(kStageForce);
     last_two_scale = two_scale;
     keys_valid = true;
@@ -657,11 +669,14 @@ sph_status Engine::set_tuning(const sph_tuning& t_in) {
 }
 
 // Times the variants of the density and force kernels on the current sorted
-// state (the inputs of the last step): every lanes-per-particle variant of
-// each, and the hit-mask pair with every hit-list capacity.  Keeps the
-// fastest density + force combination and re-runs both with it, so the state
-// is what the last step would have produced with it.  Both kernels only read
-// the sorted buffers, so repeating them is safe.
+// state (the inputs of the last step), each as a step like the last one would
+// run it: every lanes-per-particle variant of each pass (one lane in both
+// passes as a pair, where the masks pair stands in for them), and the hit-mask
+// pair with every hit-list capacity; sizes that run in teams have one form of
+// either and keep the list and block they are set to.  Keeps the fastest
+// density + force combination and re-runs both with it, so the state is what
+// the last step would have produced with it.  Both kernels only read the
+// sorted buffers, so repeating them is safe.
 sph_status Engine::autotune(int reps, sph_tuning* out) {
     if (reps < 1) return fail(SPH_INVALID_ARG, "reps must be >= 1");
     if (!keys_valid) return fail(SPH_INVALID_ARG, "autotune needs the state of one step: advance once first");
@@ -674,11 +689,9 @@ sph_status Engine::autotune(int reps, sph_tuning* out) {
         if (st != SPH_OK) return st;
         bytes += sizeof(uint64_t) * row_words_u64(N);
     }
-    StepBuffers plain = buffers();
-    plain.masks = nullptr;
-    if (last_two_scale && ts) plain.state_b = twoscale_final_state(*this);
-    StepBuffers withm = plain;
-    withm.masks = masks;
+    const bool two_scale = last_two_scale && ts;
+    StepBuffers base = buffers();
+    if (two_scale) base.state_b = twoscale_final_state(*this);
     const OnDevice on(device);
     hipEvent_t e0 = nullptr, e1 = nullptr;
     if (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess) {
@@ -686,7 +699,10 @@ sph_status Engine::autotune(int reps, sph_tuning* out) {
         return fail(SPH_DEVICE_ERROR, "event creation failed");
     }
     bool ok = true;
-    auto time_it = [&](auto&& run) -> float {
+    auto time_it = [&](const sph_tuning& t, bool density, bool force) -> float {
+        StepBuffers b = base;
+        route(b, t, two_scale);
+        auto run = [&] { launch_passes(stream, b, t, density, force); };
         run();  // warm-up
         (void)hipEventRecord(e0, stream);
         for (int r = 0; r < reps; ++r) run();
@@ -699,58 +715,70 @@ sph_status Engine::autotune(int reps, sph_tuning* out) {
         (void)hipEventElapsedTime(&ms, e0, e1);
         return ms;
     };
-    // block sizes apply to the one-lane and hit-mask variants (the
-    // cooperative ones keep 256 threads): one block size for the pair
+    sph_tuning pick = tuning;
+    float best = 1e30f;
+    auto offer = [&](const sph_tuning& t, float ms) {
+        if (ms < best) {
+            best = ms;
+            pick = t;
+        }
+    };
     static const int cand[] = {1, 2, 4, 8, 16};
     static const int caps[] = {32, 40, 48, 64};
-    static const int blks[] = {128, 256};
-    sph_tuning pick = tuning;
-    float best_plain = 1e30f, best_masks = 1e30f;
-    sph_tuning pick_plain = tuning, pick_masks = tuning;
-    for (int B : blks) {
-        float best_d = 1e30f, best_f = 1e30f;
-        int ld = 1, lf = 1;
-        for (int L : cand) {
-            if (L > 1 && B != 256) continue;
-            float ms = time_it([&] { launch_density(stream, plain, L, B); });
-            if (ms < best_d) { best_d = ms; ld = L; }
+    static const int blks[] = {256, 128};
+    // without masks: a pass's time with L lanes does not depend on the other's
+    float td[17], tf[17];
+    for (int L : cand) {
+        sph_tuning t = tuning;
+        t.hit_masks = 0;
+        t.block = 256;
+        t.density_lanes = L;
+        t.force_lanes = 2;
+        td[L] = time_it(t, true, false);
+        t.density_lanes = 2;
+        t.force_lanes = L;
+        tf[L] = time_it(t, false, true);
+    }
+    const bool teams = team_size(N, false), team_masks = team_size(N, true) && !two_scale;
+    for (int ld : cand)
+        for (int lf : cand) {
+            sph_tuning t = tuning;
+            t.hit_masks = 0;
+            t.density_lanes = ld;
+            t.force_lanes = lf;
+            if (!teams) t.block = 256;
+            if (ld == 1 && lf == 1 && one_lane_by_masks(t, two_scale)) offer(t, time_it(t, true, true));
+            else offer(t, td[ld] + tf[lf]);
         }
-        for (int L : cand) {
-            if (L > 1 && B != 256) continue;
-            float ms = time_it([&] { launch_force(stream, plain, L, B); });
-            if (ms < best_f) { best_f = ms; lf = L; }
-        }
-        if (best_d + best_f < best_plain) {
-            best_plain = best_d + best_f;
-            pick_plain.density_lanes = ld;
-            pick_plain.force_lanes = lf;
-            pick_plain.block = B;
-        }
-        float t_dm = time_it([&] { launch_density(stream, withm, 1, B); });
-        for (int c : caps) {
-            float ms = time_it([&] { launch_force(stream, withm, c, B); });
-            if (t_dm + ms < best_masks) {
-                best_masks = t_dm + ms;
-                pick_masks.hit_list = c;
-                pick_masks.block = B;
+    // the loops with smaller blocks (cooperative variants keep 256 threads,
+    // teams and the masks pair for the loops theirs)
+    sph_tuning one = tuning;
+    one.hit_masks = 0;
+    one.density_lanes = one.force_lanes = 1;
+    one.block = 128;
+    if (!teams && !one_lane_by_masks(one, two_scale)) offer(one, time_it(one, true, true));
+    sph_tuning hm = tuning;
+    hm.hit_masks = 1;
+    if (team_masks) {
+        offer(hm, time_it(hm, true, true));
+    } else {
+        for (int B : blks) {
+            hm.block = B;
+            const float t_d = time_it(hm, true, false);
+            for (int c : caps) {
+                hm.hit_list = c;
+                offer(hm, t_d + time_it(hm, false, true));
             }
         }
     }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     if (!ok) return fail(SPH_DEVICE_ERROR, "autotune: kernel failed");
-    if (best_masks < best_plain) {
-        pick = pick_masks;
-        pick.hit_masks = 1;
-    } else {
-        pick = pick_plain;
-        pick.hit_masks = 0;
-    }
     sph_status st = set_tuning(pick);
     if (st != SPH_OK) return st;
-    StepBuffers& b = tuning.hit_masks ? withm : plain;
-    launch_density(stream, b, tuning.density_lanes, tuning.block);
-    launch_force(stream, b, tuning.hit_masks ? tuning.hit_list : tuning.force_lanes, tuning.block);
+    StepBuffers b = base;
+    route(b, tuning, two_scale);
+    launch_passes(stream, b, tuning, true, true);
     st = check_launch("autotune");
     if (st != SPH_OK) return st;
     if (out) *out = tuning;

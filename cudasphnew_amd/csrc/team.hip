@@ -342,7 +342,7 @@ constexpr uint32_t kTeamMax = 40960, kTeamMaxMasks = 28672;
 
 bool team_size(uint32_t n, bool masks) { return n <= (masks ? kTeamMaxMasks : kTeamMax); }
 
-bool team_step(const StepBuffers& b) { return team_size(b.n, b.masks != nullptr) && !b.split.state; }
+bool team_step(const StepBuffers& b) { return b.teams && team_size(b.n, b.masks != nullptr); }
 
 void launch_density_team(hipStream_t st, const StepBuffers& b) {
     const bool one = b.nscenes == 1;

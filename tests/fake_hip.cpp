@@ -52,6 +52,14 @@ long long fake_count(const char* name) {
     std::lock_guard<std::mutex> g(lock);
     return counters[name];
 }
+// launches of the kernels whose mangled names hold `part`
+long long fake_launches(const char* part) {
+    std::lock_guard<std::mutex> g(lock);
+    long long n = 0;
+    for (auto& c : counters)
+        if (c.first.compare(0, 8, "mangled ") == 0 && c.first.find(part) != std::string::npos) n += c.second;
+    return n;
+}
 void fake_fail(const char* name, long long after) { fail_from[name] = after; }
 void fake_work(const char* name) { fail_from.erase(name); }
 void fake_free_bytes(size_t n) { free_bytes = n; }
@@ -251,6 +259,7 @@ int hipLaunchKernel(const void* f, Dim3, Dim3, void** args, size_t, void*) {
     const size_t at = m.find("k_");
     const std::string name = at == std::string::npos ? m : m.substr(at, m.find_first_of("IE", at) - at);
     count("kernel " + name);
+    count("mangled " + m);
     count("kernels");
     if (name == "k_read_xyz") {
         const uint32_t n = *static_cast<uint32_t*>(args[0]);

@@ -16,6 +16,8 @@ fake = C.CDLL({lib!r}, mode=C.RTLD_GLOBAL)
 fake.fake_count.restype = C.c_longlong
 fake.fake_free_bytes.argtypes = [C.c_size_t]
 fake.fake_fail.argtypes = [C.c_char_p, C.c_longlong]
+fake.fake_launches.restype = C.c_longlong
+launches = lambda part: fake.fake_launches(part.encode())
 count = lambda name: fake.fake_count(name.encode())
 import numpy as np
 import cudasphnew_amd as S
