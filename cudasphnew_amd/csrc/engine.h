@@ -118,6 +118,11 @@ struct Engine {
     uint64_t* masks = nullptr;   // row words [9][N] + chunk masks [3][9][N] (common.h)
     // the masks pair stands in for the one-lane variants t in such a step
     bool one_lane_by_masks(const sph_tuning& t, bool two_scale) const;
+    // its masks, while nothing else has asked for them
+    bool masks_lent = false, masks_refused = false;
+    void lend_masks();
+    void return_masks();
+    sph_status need_masks();
     // sets what selects the two passes' kernels under variants t
     void route(StepBuffers& b, const sph_tuning& t, bool two_scale) const;
 

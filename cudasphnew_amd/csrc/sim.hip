@@ -260,20 +260,7 @@ sph_status Engine::init(int S, const sph_params* P, const sph_scene* scenes) {
         bytes += sorter.bytes();
     }
 
-    // the one-lane variants' masks (one_lane_by_masks): 180 bytes a particle,
-    // unless they are more than an eighth of the free memory; without them
-    // the loops run
-    if (one_lane_by_masks(tuning, false)) {
-        size_t free_bytes = 0, total = 0;
-        const size_t need = sizeof(uint64_t) * row_words_u64(N);
-        if (hipMemGetInfo(&free_bytes, &total) == hipSuccess && need <= free_bytes / 8 &&
-            hipMalloc(&masks, need) == hipSuccess) {
-            bytes += need;
-        } else {
-            (void)hipGetLastError();
-            masks = nullptr;
-        }
-    }
+    lend_masks();
 
     // host staging, then upload
     std::vector<float4> hp(N), hv(N), g4;
@@ -406,6 +393,48 @@ bool Engine::one_lane_by_masks(const sph_tuning& t, bool two_scale) const {
            !team_size(N, true);
 }
 
+// The masks of that pair: 180 bytes a particle, unless they are more than an
+// eighth of the free memory; without them the loops run.  Taken with the
+// handle (a first step with an allocation in it is slower), given back when
+// other variants or two-scale steps leave them unread, and taken again by the
+// next step that reads them.
+void Engine::lend_masks() {
+    if (masks || masks_refused || !one_lane_by_masks(tuning, false)) return;
+    const OnDevice on(device);
+    // a step may come while the thread captures another stream
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    size_t free_bytes = 0, total = 0;
+    const size_t need = sizeof(uint64_t) * row_words_u64(N);
+    if (hipMemGetInfo(&free_bytes, &total) == hipSuccess && need <= free_bytes / 8 &&
+        hipMalloc(reinterpret_cast<void**>(&masks), need) == hipSuccess) {
+        bytes += need;
+        masks_lent = true;
+        drop_graph();
+    } else {
+        (void)hipGetLastError();
+        masks = nullptr;
+        masks_refused = true;
+    }
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+}
+
+void Engine::return_masks() {
+    if (!masks_lent) return;
+    (void)hipStreamSynchronize(stream);
+    drop_graph();
+    (void)hipFree(masks);
+    bytes -= sizeof(uint64_t) * row_words_u64(N);
+    masks = nullptr;
+    masks_lent = false;
+}
+
+// The masks of the hit-mask variants: kept from here on.
+sph_status Engine::need_masks() {
+    masks_lent = false;
+    return masks ? SPH_OK : alloc(&masks, row_words_u64(N));
+}
+
 // The kernels of a step's density and force passes under variants t; the
 // autotuner times what this selects.
 void Engine::route(StepBuffers& b, const sph_tuning& t, bool two_scale) const {
@@ -473,7 +502,9 @@ sph_status Engine::step(int n, bool two_scale) {
         sph_status st = twoscale_create(*this);
         if (st != SPH_OK) return st;
         drop_graph();   // the step's buffers now include the sub-particle pass's
+        return_masks();
     }
+    if (!two_scale && n > 0) lend_masks();
     for (int i = 0; i < n; ++i) {
         if (retune_every && keys_valid && steps > 0 && steps % retune_every == 0) {
             sph_status st = autotune(2, nullptr);
@@ -656,15 +687,17 @@ sph_status Engine::set_tuning(const sph_tuning& t_in) {
         return fail(SPH_INVALID_ARG, "lanes per particle must be 1, 2, 4, 8 or 16");
     if (t.hit_masks != 0 && t.hit_masks != 1) return fail(SPH_INVALID_ARG, "hit_masks must be 0 or 1");
     if (!list_ok(t.hit_list)) return fail(SPH_INVALID_ARG, "hit_list must be 32, 40, 48 or 64");
-    if (t.hit_masks && !masks) {
-        sph_status st = alloc(&masks, row_words_u64(N));
+    if (t.hit_masks) {
+        sph_status st = need_masks();
         if (st != SPH_OK) return st;
-        bytes += sizeof(uint64_t) * row_words_u64(N);
+    } else if (!one_lane_by_masks(t, false)) {
+        return_masks();
     }
     if (t.density_lanes != tuning.density_lanes || t.force_lanes != tuning.force_lanes ||
         t.hit_masks != tuning.hit_masks || t.hit_list != tuning.hit_list || t.block != tuning.block)
         drop_graph();
     tuning = t;
+    masks_refused = false;
     return SPH_OK;
 }
 
@@ -684,11 +717,7 @@ sph_status Engine::autotune(int reps, sph_tuning* out) {
         sph_status st = resolve_timing();
         if (st != SPH_OK) return st;
     }
-    if (!masks) {
-        sph_status st = alloc(&masks, row_words_u64(N));
-        if (st != SPH_OK) return st;
-        bytes += sizeof(uint64_t) * row_words_u64(N);
-    }
+    if (sph_status st = need_masks(); st != SPH_OK) return st;
     const bool two_scale = last_two_scale && ts;
     StepBuffers base = buffers();
     if (two_scale) base.state_b = twoscale_final_state(*this);
