@@ -102,12 +102,16 @@ struct Engine {
     hipEvent_t next_event();
     sph_status resolve_timing();
 
-    // graph capture of the steady-state step, plain and two-scale
+    // graph capture of the steady-state plain step
     bool use_graph = false;
     uint32_t retune_every = 0;   // re-run the autotuner before every n-th step (0: never)
     static constexpr int kGraphSizes = 3;
     hipGraph_t graph[kGraphSizes] = {};           // of 2^k steps
     hipGraphExec_t graph_exec[kGraphSizes] = {};
+    // when a longer graph is built: steps left of a call, or replayed before it
+    static constexpr int kGraphPays = 16;
+    static constexpr uint32_t kGraphSettled = 8;
+    uint32_t replayed = 0;                        // steps since the last drop
 
     TwoScale* ts = nullptr;
     bool last_two_scale = false;

@@ -505,6 +505,7 @@ sph_status Engine::step(int n, bool two_scale) {
         return_masks();
     }
     if (!two_scale && n > 0) lend_masks();
+    const bool settled = replayed >= kGraphSettled;
     for (int i = 0; i < n; ++i) {
         if (retune_every && keys_valid && steps > 0 && steps % retune_every == 0) {
             sph_status st = autotune(2, nullptr);
@@ -521,12 +522,16 @@ sph_status Engine::step(int n, bool two_scale) {
             // the distance to the next retuning: the device idles 8 us
             // between replays.  Four steps and a position export, graphs of
             // one step only and these: 180 / 159 us at 16,384 particles, 273
-            // / 249 at 120,000, 869 / 851 at 1M; graphs of eight gain 2% more
-            // on the smallest sets
+            // / 249 at 120,000; graphs of eight gain 2% more on the smallest
+            // sets.  A longer graph takes the host 60 to 100 us to build, as
+            // much as it saves in 16 steps: it is built for a call with so
+            // many left, or once calls before this one have replayed some
+            // since the last change of what a step launches
             int left = n - i;
             if (retune_every) left = std::min(left, (int)(retune_every - steps % retune_every));
-            int k = 0;
-            while (k + 1 < kGraphSizes && 2 << k <= left) ++k;
+            const bool build = left >= kGraphPays || settled;
+            int k = kGraphSizes - 1;
+            while (k > 0 && (1 << k > left || !(build || graph_exec[k]))) --k;
             hipGraph_t& g = graph[k];
             hipGraphExec_t& gx = graph_exec[k];
             if (!gx) {
@@ -540,6 +545,7 @@ sph_status Engine::step(int n, bool two_scale) {
             }
             if (hipGraphLaunch(gx, stream) != hipSuccess)
                 return fail(SPH_DEVICE_ERROR, "hipGraphLaunch failed");
+            replayed += 1u << k;
             steps += (1 << k) - 1;
             i += (1 << k) - 1;
             last_two_scale = two_scale;
@@ -668,6 +674,7 @@ sph_status Engine::own_distance() {
 }
 
 void Engine::drop_graph() {
+    replayed = 0;
     for (int k = 0; k < kGraphSizes; ++k) {
         if (graph_exec[k]) (void)hipGraphExecDestroy(graph_exec[k]);
         if (graph[k]) (void)hipGraphDestroy(graph[k]);

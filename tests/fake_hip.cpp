@@ -198,11 +198,14 @@ int hipEventElapsedTime(float* ms, void*, void*) {
     return 0;
 }
 int hipThreadExchangeStreamCaptureMode(int*) { return 0; }
+thread_local bool capturing = false;
 int hipStreamBeginCapture(void*, int) {
     count("capture");
+    capturing = true;
     return 0;
 }
 int hipStreamEndCapture(void*, void** g) {
+    capturing = false;
     *g = new Object{current};
     return 0;
 }
@@ -260,7 +263,7 @@ int hipLaunchKernel(const void* f, Dim3, Dim3, void** args, size_t, void*) {
     const std::string name = at == std::string::npos ? m : m.substr(at, m.find_first_of("IE", at) - at);
     count("kernel " + name);
     count("mangled " + m);
-    count("kernels");
+    count(capturing ? "captured" : "kernels");
     if (name == "k_read_xyz") {
         const uint32_t n = *static_cast<uint32_t*>(args[0]);
         const float* src = *static_cast<float**>(args[1]);
