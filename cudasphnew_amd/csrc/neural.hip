@@ -105,13 +105,15 @@ __device__ __forceinline__ f32x4 mfma(bf16x8 a, bf16x8 b, f32x4 c) {
 }
 
 // 1 / (1 + exp(-z)).  One Newton step on the hardware reciprocal of a number
-// in [1, 2^126] is the correctly rounded quotient (checked against 1.0f / d
-// over every mantissa of the binades), in half the division's operations; past
-// 2^126 (z < -87) the result stays at 2^-126.
+// of at most 2^126 gives the quotient that the division rounds to, in half the
+// operations.  The denominator is at least 1 and taken 2^32 times smaller, so
+// that only an infinite one (z < -88.7) meets the bound, and the quotient's own
+// factor 2^-32 makes that 0 and the ones below the normal numbers what they
+// are; a NaN in z is left to the products with z.
 __device__ __forceinline__ float sigmoid(float z) {
-    const float d = fminf(1.0f + __expf(-z), 0x1p126f);
+    const float d = fminf(fmaf(__expf(-z), 0x1p-32f, 0x1p-32f), 0x1p126f);
     const float r = __builtin_amdgcn_rcpf(d);
-    return fmaf(fmaf(-d, r, 1.0f), r, r);
+    return fmaf(fmaf(-d, r, 1.0f), r, r) * 0x1p-32f;
 }
 
 // sin(pi x) and cos(pi x): exact reduction to r = x - 2 rint(x/2) in
