@@ -169,6 +169,14 @@ __device__ __forceinline__ uint32_t sub_cell_key(const DevScene& S, float x, flo
     return (uint32_t)(S.snx * (S.sny * cz + cy) + cx);
 }
 
+// LDS written by lanes of a wavefront is read by its other lanes: in program
+// order, no barrier needed beyond keeping the compiler from moving accesses.
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // XCD-aware block order.  The 8 XCDs of an MI355X receive workgroups
 // round-robin (block b runs on XCD b % 8), each XCD with its own L2.  Giving
 // XCD x the contiguous logical blocks [x*G/8, (x+1)*G/8) keeps neighbouring

@@ -510,14 +510,6 @@ __device__ __forceinline__ uint32_t density_row(Row at, int cnt, float4 xi, floa
     return m;
 }
 
-// LDS written by lanes of a wavefront is read by its other lanes: in program
-// order, no barrier needed beyond keeping the compiler from moving accesses.
-__device__ __forceinline__ void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // The nine rows of a particle's neighbour range one after the other, plane by
 // plane: the lane's slot run of row (dk, dj) as row_slots finds it.  What does
 // not depend on the row is formed once (the table indices of the run's cells,
@@ -900,9 +892,9 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(CAP <= 40 ? 5
 }
 
 // A field of one scene in original-id order, as a host read wants it: the
-// device scatters by id (a few us at 256,000 particles), so that the copy to
-// the host is the field alone, straight into the caller's array.  Before, the
-// float4 records and the ids were copied and the host scattered them.
+// device scatters by id (a few us at 256,000 particles), so that what crosses
+// to the host (HostCopy's pinned slots) is the field alone.  Before, the float4
+// records and the ids were copied and the host scattered them.
 __global__ __launch_bounds__(kBlock) void k_read_xyz(uint32_t n, const float4* __restrict__ src,
                                                      const uint32_t* __restrict__ oid, float* __restrict__ out) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;

@@ -13,9 +13,10 @@
 // 128 -> 64 -> 64 -> 64 (SiLU) -> 1; d = out_scale * y.
 //
 // MFMA operand layout (16x16x32 bf16): lane l holds A[l%16][8(l/16)+0..7],
-// B[8(l/16)+0..7][l%16] and produces D[4(l/16)+j][l%16], j < 4.  A tile of 64
-// samples is worked by four wavefronts, wave w owning sample rows 16w..16w+15
-// of every row-parallel product.
+// B[8(l/16)+0..7][l%16] and produces D[4(l/16)+j][l%16], j < 4.  Evaluation
+// and the step's normals work tiles of 64 points with four wavefronts, wave w
+// owning points 16w..16w+15, the points on the rows; training works tiles of
+// 128 samples with eight wavefronts, the samples on the columns.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -125,16 +126,6 @@ __device__ __forceinline__ void sincospi_hw(float x, float& s, float& c) {
     c = __builtin_amdgcn_cosf(t);
 }
 
-// Feature f of normalized coordinates u.
-__device__ __forceinline__ float feature(const NetView& net, int f, const float u[3]) {
-    if (f < 3) return u[f];
-    if (f >= kFeat) return 0.0f;
-    int i = f - 3, k = i / 6, a = (i % 6) >> 1;
-    float s, c;
-    sincospi_hw(net.freq[k] * u[a], s, c);
-    return (i & 1) ? c : s;
-}
-
 // d feature f / d u_a(f) (the axis it depends on is returned in axis).
 __device__ __forceinline__ float feature_du(const NetView& net, int f, const float u[3], int& axis) {
     if (f < 3) {
@@ -176,37 +167,43 @@ __device__ __forceinline__ void rows_x_wt(const uint16_t* sA, const uint16_t* __
     }
 }
 
-// Input layer of a tile: features of sample row 16w + lane%16 computed in
-// registers in A-fragment form (k = 32ks + 8(lane/16) + 0..7).  Optionally
-// also stored transposed ([k][s]) for the weight-gradient product.
-__device__ __forceinline__ void input_layer(const NetView& net, const float u[3], int lane, int w, f32x4 acc[4],
-                                            uint16_t* sA0T) {
+__device__ __forceinline__ uint2 pack4(float a, float b, float c, float d) {
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    const f32x2 lo = {a, b}, hi = {c, d};
+    return make_uint2(__builtin_bit_cast(uint32_t, __builtin_convertvector(lo, bf16x2)),
+                      __builtin_bit_cast(uint32_t, __builtin_convertvector(hi, bf16x2)));
+}
+
+// Features k0 .. k0 + 7, k0 = 8 (4 ks + lane / 16), of normalized coordinates
+// u, packed as BF16.
+__device__ __forceinline__ uint4 feature_frag(const NetView& net, const float u[3], int ks, int lane) {
+    // features f0..f0+7 (f0 = 8q) use the (sin, cos) pairs
+    // m = 4q - 2 .. 4q + 2 (pair m = 3k + a: features 3 + 2m, 4 + 2m)
+    const int q = 4 * ks + (lane >> 4), f0 = 8 * q;
+    float ps[5], pc[5];
+#pragma unroll
+    for (int t = 0; t < 5; ++t) {
+        const int m = 4 * q - 2 + t;
+        ps[t] = pc[t] = 0.0f;
+        if (m >= 0 && m < 3 * kFreqs) sincospi_hw(net.freq[m / 3] * u[m % 3], ps[t], pc[t]);
+    }
+    float v[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const int f = f0 + j, t = (j + 1) >> 1;
+        v[j] = f < 3 ? u[f < 3 ? f : 0] : (f >= kFeat ? 0.0f : ((j & 1) ? ps[t] : pc[t]));
+    }
+    const uint2 a = pack4(v[0], v[1], v[2], v[3]), b = pack4(v[4], v[5], v[6], v[7]);
+    return make_uint4(a.x, a.y, b.x, b.y);
+}
+
+// Input layer of a tile: features of point row 16w + lane%16 computed in
+// registers in A-fragment form (k = 32ks + 8(lane/16) + 0..7).
+__device__ __forceinline__ void input_layer(const NetView& net, const float u[3], int lane, int w, f32x4 acc[4]) {
 #pragma unroll
     for (int ks = 0; ks < kK1 / 32; ++ks) {
-        // features f0..f0+7 (f0 = 8q) use the (sin, cos) pairs
-        // m = 4q - 2 .. 4q + 2 (pair m = 3k + a: features 3 + 2m, 4 + 2m)
-        const int q = 4 * ks + (lane >> 4), f0 = 8 * q;
-        float ps[5], pc[5];
-#pragma unroll
-        for (int t = 0; t < 5; ++t) {
-            const int m = 4 * q - 2 + t;
-            ps[t] = pc[t] = 0.0f;
-            if (m >= 0 && m < 3 * kFreqs) sincospi_hw(net.freq[m / 3] * u[m % 3], ps[t], pc[t]);
-        }
-        uint16_t v[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const int f = f0 + j, t = (j + 1) >> 1;
-            const float g = f < 3 ? u[f < 3 ? f : 0] : (f >= kFeat ? 0.0f : ((j & 1) ? ps[t] : pc[t]));
-            v[j] = f2bf(g);
-            if (sA0T) sA0T[f * kLds + 16 * w + (lane & 15)] = v[j];
-        }
-        uint4 pk;
-        pk.x = v[0] | ((uint32_t)v[1] << 16);
-        pk.y = v[2] | ((uint32_t)v[3] << 16);
-        pk.z = v[4] | ((uint32_t)v[5] << 16);
-        pk.w = v[6] | ((uint32_t)v[7] << 16);
-        bf16x8 a = __builtin_bit_cast(bf16x8, pk);
+        const bf16x8 a = __builtin_bit_cast(bf16x8, feature_frag(net, u, ks, lane));
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
             bf16x8 b = frag_ld(net.w.W1T + (size_t)(16 * c + (lane & 15)) * kK1 + 32 * ks + 8 * (lane >> 4));
@@ -216,9 +213,9 @@ __device__ __forceinline__ void input_layer(const NetView& net, const float u[3]
 }
 
 // Bias + SiLU of a 64-wide layer output held in D layout; writes the BF16
-// activation (row-major and, optionally, transposed) and keeps silu'(z).
+// activation (row-major) and keeps silu'(z).
 __device__ __forceinline__ void activate(const float* __restrict__ bias, f32x4 acc[4], f32x4 dact[4], int lane,
-                                         int w, uint16_t* sA, uint16_t* sAT, float* a_out = nullptr) {
+                                         int w, uint16_t* sA, float* a_out = nullptr) {
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
         int n = 16 * c + (lane & 15);
@@ -231,35 +228,34 @@ __device__ __forceinline__ void activate(const float* __restrict__ bias, f32x4 a
             float a = z * sg;
             dact[c][j] = sg * (1.0f + z * (1.0f - sg));
             if (a_out) a_out[4 * c + j] = a;
-            uint16_t ab = f2bf(a);
-            if (sA) sA[s * kLds + n] = ab;
-            if (sAT) sAT[n * kLds + s] = ab;
+            if (sA) sA[s * kLds + n] = f2bf(a);
         }
     }
 }
 
-// Writes a back-propagated dz (D layout, FP32) as BF16, row-major and
-// transposed.
-__device__ __forceinline__ void store_dz(const f32x4 dz[4], int lane, int w, uint16_t* sdZ, uint16_t* sdZT) {
+// Writes a back-propagated dz (D layout, FP32) as BF16, row-major.
+__device__ __forceinline__ void store_dz(const f32x4 dz[4], int lane, int w, uint16_t* sdZ) {
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
         int n = 16 * c + (lane & 15);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            int s = 16 * w + 4 * (lane >> 4) + j;
-            uint16_t v = f2bf(dz[c][j]);
-            sdZ[s * kLds + n] = v;
-            if (sdZT) sdZT[n * kLds + s] = v;
-        }
+        for (int j = 0; j < 4; ++j) sdZ[(16 * w + 4 * (lane >> 4) + j) * kLds + n] = f2bf(dz[c][j]);
     }
 }
 
-// Sum over the 16 lanes that share lane/16 (one sample row group).
-__device__ __forceinline__ float row_sum16(float v) {
-    v += __shfl_xor(v, 1, 64);
-    v += __shfl_xor(v, 2, 64);
-    v += __shfl_xor(v, 4, 64);
-    v += __shfl_xor(v, 8, 64);
+// Lane permutations inside 16 lanes, one VALU operation each (DPP).
+template <int CTRL>
+__device__ __forceinline__ float dpp(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, true));
+}
+constexpr int kDppXor1 = 0xB1, kDppXor3 = 0x1B, kDppXor7 = 0x141, kDppXor15 = 0x140;   // lane ^ 1, 3, 7, 15
+
+// Sum of a lane's value over the 16 lanes of its lane / 16 group.
+__device__ __forceinline__ float sum16(float v) {
+    v += dpp<kDppXor1>(v);
+    v += dpp<kDppXor3>(v);
+    v += dpp<kDppXor7>(v);
+    v += dpp<kDppXor15>(v);
     return v;
 }
 
@@ -288,21 +284,6 @@ constexpr int kPartStride = (kParams + 3) / 4 * 4;
 static_assert(ob1 % 4 == 0 && oW2 % 4 == 0 && ob2 % 4 == 0 && oW3 % 4 == 0 && ob3 % 4 == 0 && ow4 % 4 == 0 &&
                   ob4 % 4 == 0,
               "sections are read four values at a time");
-
-__device__ __forceinline__ uint2 pack4(float a, float b, float c, float d) {
-    typedef float f32x2 __attribute__((ext_vector_type(2)));
-    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-    const f32x2 lo = {a, b}, hi = {c, d};
-    return make_uint2(__builtin_bit_cast(uint32_t, __builtin_convertvector(lo, bf16x2)),
-                      __builtin_bit_cast(uint32_t, __builtin_convertvector(hi, bf16x2)));
-}
-
-// LDS written by lanes of a wavefront and read by its other lanes.
-__device__ __forceinline__ void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 
 // Fragment of a sample-major LDS tile read transposed: element e of lane l is
 // tile[row0 + 8 (l / 16) + e][col0 + l % 16].  ds_read_b64_tr_b16 works on 16
@@ -346,29 +327,6 @@ __device__ __forceinline__ void stage(const uint16_t* __restrict__ W, uint16_t* 
     }
 }
 
-// Features k0 .. k0 + 7, k0 = 8 (4 ks + lane / 16), of normalized coordinates
-// u, packed as BF16.
-__device__ __forceinline__ uint4 feature_frag(const NetView& net, const float u[3], int ks, int lane) {
-    // features f0..f0+7 (f0 = 8q) use the (sin, cos) pairs
-    // m = 4q - 2 .. 4q + 2 (pair m = 3k + a: features 3 + 2m, 4 + 2m)
-    const int q = 4 * ks + (lane >> 4), f0 = 8 * q;
-    float ps[5], pc[5];
-#pragma unroll
-    for (int t = 0; t < 5; ++t) {
-        const int m = 4 * q - 2 + t;
-        ps[t] = pc[t] = 0.0f;
-        if (m >= 0 && m < 3 * kFreqs) sincospi_hw(net.freq[m / 3] * u[m % 3], ps[t], pc[t]);
-    }
-    float v[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-        const int f = f0 + j, t = (j + 1) >> 1;
-        v[j] = f < 3 ? u[f < 3 ? f : 0] : (f >= kFeat ? 0.0f : ((j & 1) ? ps[t] : pc[t]));
-    }
-    const uint2 a = pack4(v[0], v[1], v[2], v[3]), b = pack4(v[4], v[5], v[6], v[7]);
-    return make_uint4(a.x, a.y, b.x, b.y);
-}
-
 // Bias + SiLU of a layer's outputs (acc[c][j] = output 16c + 4 (lane / 16) + j
 // of sample lane % 16); the activations replace acc, silu'(z) goes to dact and
 // the BF16 activations to the sample's LDS row (if any).
@@ -394,22 +352,6 @@ __device__ __forceinline__ void store_cols(const f32x4 v[4], int lane, uint16_t*
 #pragma unroll
     for (int c = 0; c < 4; ++c)
         *reinterpret_cast<uint2*>(row + 16 * c + 4 * (lane >> 4)) = pack4(v[c][0], v[c][1], v[c][2], v[c][3]);
-}
-
-// Lane permutations inside 16 lanes, one VALU operation each (DPP).
-template <int CTRL>
-__device__ __forceinline__ float dpp(float v) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, true));
-}
-constexpr int kDppXor1 = 0xB1, kDppXor3 = 0x1B, kDppXor7 = 0x141, kDppXor15 = 0x140;   // lane ^ 1, 3, 7, 15
-
-// Sum of a lane's value over the 16 lanes of its lane / 16 group.
-__device__ __forceinline__ float sum16(float v) {
-    v += dpp<kDppXor1>(v);
-    v += dpp<kDppXor3>(v);
-    v += dpp<kDppXor7>(v);
-    v += dpp<kDppXor15>(v);
-    return v;
 }
 
 // Sums over the 16 lanes of a lane / 16 group of the 16 values v[c][j]: lane
@@ -724,32 +666,32 @@ __device__ __forceinline__ void mlp_value_grad(const NetView& net, const float u
     f32x4 acc[4], D1[4], D2[4], D3[4];
 #pragma unroll
     for (int c = 0; c < 4; ++c) acc[c] = f32x4{0, 0, 0, 0};
-    input_layer(net, u, lane, w, acc, nullptr);
-    activate(th + ob1, acc, D1, lane, w, sA1, nullptr);
+    input_layer(net, u, lane, w, acc);
+    activate(th + ob1, acc, D1, lane, w, sA1);
     __syncthreads();
 #pragma unroll
     for (int c = 0; c < 4; ++c) acc[c] = f32x4{0, 0, 0, 0};
     rows_x_wt<kH, 4>(sA1, net.w.W2T, lane, w, acc);
-    activate(th + ob2, acc, D2, lane, w, sA2, nullptr);
+    activate(th + ob2, acc, D2, lane, w, sA2);
     __syncthreads();
 #pragma unroll
     for (int c = 0; c < 4; ++c) acc[c] = f32x4{0, 0, 0, 0};
     rows_x_wt<kH, 4>(sA2, net.w.W3T, lane, w, acc);
     float a3[16];
-    activate(th + ob3, acc, D3, lane, w, nullptr, nullptr, a3);
+    activate(th + ob3, acc, D3, lane, w, nullptr, a3);
     f32x4 dz[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         float part = 0.0f;
 #pragma unroll
         for (int c = 0; c < 4; ++c) part += a3[4 * c + j] * th[ow4 + 16 * c + (lane & 15)];
-        y[j] = row_sum16(part) + th[ob4];
+        y[j] = sum16(part) + th[ob4];
     }
 #pragma unroll
     for (int c = 0; c < 4; ++c)
 #pragma unroll
         for (int j = 0; j < 4; ++j) dz[c][j] = th[ow4 + 16 * c + (lane & 15)] * D3[c][j];
-    store_dz(dz, lane, w, sdZ, nullptr);
+    store_dz(dz, lane, w, sdZ);
     __syncthreads();
 #pragma unroll
     for (int c = 0; c < 4; ++c) acc[c] = f32x4{0, 0, 0, 0};
@@ -759,7 +701,7 @@ __device__ __forceinline__ void mlp_value_grad(const NetView& net, const float u
     for (int c = 0; c < 4; ++c)
 #pragma unroll
         for (int j = 0; j < 4; ++j) dz[c][j] = acc[c][j] * D2[c][j];
-    store_dz(dz, lane, w, sdZ, nullptr);
+    store_dz(dz, lane, w, sdZ);
     __syncthreads();
 #pragma unroll
     for (int c = 0; c < 4; ++c) acc[c] = f32x4{0, 0, 0, 0};
@@ -769,7 +711,7 @@ __device__ __forceinline__ void mlp_value_grad(const NetView& net, const float u
     for (int c = 0; c < 4; ++c)
 #pragma unroll
         for (int j = 0; j < 4; ++j) dz[c][j] = acc[c][j] * D1[c][j];
-    store_dz(dz, lane, w, sdZ, nullptr);
+    store_dz(dz, lane, w, sdZ);
     __syncthreads();
     // dy/dg = dz1 . W1^T (64 x 128), then dy/du through the feature map
     f32x4 dg[8];
@@ -793,9 +735,9 @@ __device__ __forceinline__ void mlp_value_grad(const NetView& net, const float u
             gu[j][1] += axis == 1 ? v : 0.0f;
             gu[j][2] += axis == 2 ? v : 0.0f;
         }
-        gu[j][0] = row_sum16(gu[j][0]);
-        gu[j][1] = row_sum16(gu[j][1]);
-        gu[j][2] = row_sum16(gu[j][2]);
+        gu[j][0] = sum16(gu[j][0]);
+        gu[j][1] = sum16(gu[j][1]);
+        gu[j][2] = sum16(gu[j][2]);
     }
 }
 
@@ -810,25 +752,25 @@ __device__ __forceinline__ void mlp_value(const NetView& net, const float u[3], 
     __syncthreads();
 #pragma unroll
     for (int c = 0; c < 4; ++c) acc[c] = f32x4{0, 0, 0, 0};
-    input_layer(net, u, lane, w, acc, nullptr);
-    activate(th + ob1, acc, dact, lane, w, sA1, nullptr);
+    input_layer(net, u, lane, w, acc);
+    activate(th + ob1, acc, dact, lane, w, sA1);
     __syncthreads();
 #pragma unroll
     for (int c = 0; c < 4; ++c) acc[c] = f32x4{0, 0, 0, 0};
     rows_x_wt<kH, 4>(sA1, net.w.W2T, lane, w, acc);
-    activate(th + ob2, acc, dact, lane, w, sA2, nullptr);
+    activate(th + ob2, acc, dact, lane, w, sA2);
     __syncthreads();
 #pragma unroll
     for (int c = 0; c < 4; ++c) acc[c] = f32x4{0, 0, 0, 0};
     rows_x_wt<kH, 4>(sA2, net.w.W3T, lane, w, acc);
     float a3[16];
-    activate(th + ob3, acc, dact, lane, w, nullptr, nullptr, a3);
+    activate(th + ob3, acc, dact, lane, w, nullptr, a3);
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         float part = 0.0f;
 #pragma unroll
         for (int c = 0; c < 4; ++c) part += a3[4 * c + j] * th[ow4 + 16 * c + (lane & 15)];
-        y[j] = row_sum16(part) + th[ob4];
+        y[j] = sum16(part) + th[ob4];
     }
 }
 

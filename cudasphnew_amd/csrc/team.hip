@@ -29,14 +29,6 @@ constexpr int kRow = 32;                     // candidates of a row on the fast 
 constexpr int kList = 9 * kRow;              // list entries per team: every candidate of the fast path
 constexpr int kPad = kList + kTeam;          // + the zero padding of a partial vector read
 
-// LDS written by lanes of a wavefront is read by its other lanes: in program
-// order, no barrier needed beyond keeping the compiler from moving accesses.
-__device__ __forceinline__ void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // The nine rows' runs of a team's particle: lane r < 9 finds row r, then all
 // lanes hold all rows.  b and cnt are indexed with constants only (a loop
 // over them that stays a loop puts both in scratch memory); row(r) asks lane r.

@@ -661,6 +661,7 @@ __global__ __launch_bounds__(kB) void k_ts_density(const TSCounts* __restrict__ 
         // reads in place of one a row (30.7 -> 22.9 us for 111,000
         // sub-particles; loading the next row's candidates early takes 42: the
         // loads past a row's end cost more than the wait)
+        static_assert(kTsLanes == 4, "nine rows in three rounds of lanes");
         int rb[3], re[3];
         {
             const SubRows R = sub_rows(S, xi);
