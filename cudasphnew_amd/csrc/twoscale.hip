@@ -1000,13 +1000,16 @@ sph_status twoscale_create(Engine& e) {
     e.ts = t;   // owned by the engine from here on (freed by twoscale_destroy)
     if (!ok) {
         (void)hipGetLastError();
+        twoscale_destroy(e);   // a later step starts from nothing
         return e.fail(SPH_OUT_OF_MEMORY, "two-scale buffers");
     }
     t->bytes += t->use_cell_sort ? t->csort.bytes : t->sorter.bytes();
     if (hipMemset(t->srange, 0xFF, (size_t)t->sub_cells * sizeof(int2)) != hipSuccess ||
         hipMemset(t->counts, 0, sizeof(TSCounts)) != hipSuccess ||
-        hipMemset(t->state_fin, 0, e.N) != hipSuccess || hipDeviceSynchronize() != hipSuccess)
+        hipMemset(t->state_fin, 0, e.N) != hipSuccess || hipDeviceSynchronize() != hipSuccess) {
+        twoscale_destroy(e);
         return e.fail(SPH_DEVICE_ERROR, "two-scale initial clear");
+    }
     return SPH_OK;
 }
 
