@@ -110,7 +110,7 @@ struct Engine {
     hipGraphExec_t graph_exec[kGraphSizes] = {};
     // when a longer graph is built: steps left of a call, or replayed before it
     static constexpr int kGraphPays = 16;
-    static constexpr uint32_t kGraphSettled = 8;
+    static constexpr uint32_t kGraphSettled = 4;
     uint32_t replayed = 0;                        // steps since the last drop
 
     TwoScale* ts = nullptr;

@@ -113,8 +113,8 @@ __device__ __forceinline__ f32x4 mfma(bf16x8 a, bf16x8 b, f32x4 c) {
 // are; a NaN in z is left to the products with z.
 __device__ __forceinline__ float sigmoid(float z) {
     const float d = fminf(fmaf(__expf(-z), 0x1p-32f, 0x1p-32f), 0x1p126f);
-    const float r = __builtin_amdgcn_rcpf(d);
-    return fmaf(fmaf(-d, r, 1.0f), r, r) * 0x1p-32f;
+    const float r = __builtin_amdgcn_rcpf(d), q = r * 0x1p-32f;
+    return fmaf(fmaf(-d, r, 1.0f), q, q);
 }
 
 // sin(pi x) and cos(pi x): exact reduction to r = x - 2 rint(x/2) in
