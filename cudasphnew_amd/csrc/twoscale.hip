@@ -728,11 +728,13 @@ __global__ __launch_bounds__(kB) void k_ts_density(const TSCounts* __restrict__ 
 // a wavefront executes them as often as its lane with the most neighbours and
 // three gathers are in flight: there are two wavefronts a SIMD, and the pass is
 // bound by the latency of a lane's chain of gathers (24.5 us for 111,000
-// sub-particles one gather at a time, row by row; 14.4 now).  The rows of a
-// sub-particle with one of more than kRowMaxCands candidates are walked in
-// place.  (Before the rows kept chunks past 32 candidates, such rows were
-// tested here too: on the two-scale workload after ~1,000 steps, as the
-// flow compresses, this pass took 120 us against 44 us after.)
+// sub-particles one gather at a time, row by row; 14.4 now).  A wavefront
+// with a row of more than kRowMaxCands candidates walks all its rows in place,
+// the long ones by distance tests of 64 candidates and their hits: at four
+// times rest density (41,000 sub-particles) both sub passes take 170 us, 250
+// while the lanes with such a row walked beside the others' lists and tested
+// candidate by candidate, 263 with every row walked, one gather at a time;
+// 329,000 sub-particles: 442, 517, 494.
 constexpr int kTsForceB = 128;   // threads; the list takes 24 KiB
 constexpr int kTsCap = 48;
 
@@ -784,12 +786,13 @@ __global__ __launch_bounds__(kTsForceB) void k_ts_force(TSCounts* __restrict__ c
             cgx += wc * dx; cgy += wc * dy; cgz += wc * dz;
             cl += invj * qd * (3.0f * h2 - 7.0f * r2);
         };
-        auto pair = [&](int q) { pair_of(sp[q], sv[q]); };
-        auto near = [&](int q) {
-            const float4 xj = spos_s[q];
-            const float dx = xi.x - xj.x, dy = xi.y - xj.y, dz = xi.z - xj.z;
-            const float r2 = dx * dx + dy * dy + dz * dz;
-            return r2 <= h2 && r2 > 0.0f;
+        // the pair terms of the candidates q0 + (set bits), in order
+        auto pairs = [&](int q0, uint64_t hits) {
+            while (hits) {
+                const int q = q0 + __builtin_ctzll(hits);
+                hits &= hits - 1;
+                pair_of(sp[q], sv[q]);
+            }
         };
         // unexpanded hits: bits[row] = the rest of the current chunk's mask;
         // chunk / last: current and last chunk of each row, 2 bits per row
@@ -809,8 +812,8 @@ __global__ __launch_bounds__(kTsForceB) void k_ts_force(TSCounts* __restrict__ c
                 last |= row_last_chunk(w[row]) << (2 * row);
             }
         }
-        if (!any_long) {
-            const uint32_t* const cm = chunk_masks(smasks, cap);
+        const uint32_t* const more = chunk_masks(smasks, cap);
+        if (!__any(any_long)) {
             const int tid = threadIdx.x;
             int m;
             do {
@@ -830,7 +833,7 @@ __global__ __launch_bounds__(kTsForceB) void k_ts_force(TSCounts* __restrict__ c
                         bits[row] = lo;
                         if (lo || c == (last >> (2 * row) & 3u)) break;
                         chunk += 1u << (2 * row);   // next chunk of a long row
-                        bits[row] = cm[chunk_at(cap, c + 1, row, t)];
+                        bits[row] = more[chunk_at(cap, c + 1, row, t)];
                     }
                 }
                 if (m > 0) {
@@ -864,21 +867,28 @@ __global__ __launch_bounds__(kTsForceB) void k_ts_force(TSCounts* __restrict__ c
             for (int row = 0; row < 9; ++row) {
                 const uint64_t w = smasks[(size_t)row * cap + t];
                 if (w != kRowLong) {
-                    const uint32_t last = row_last_chunk(w);
-                    for (uint32_t ch = 0; ch <= last; ++ch) {
-                        const int b = (int)(row_first(w) + 32u * ch);
-                        uint32_t m = ch == 0 ? (uint32_t)w : chunk_masks(smasks, cap)[chunk_at(cap, ch, row, t)];
-                        while (m) {
-                            const int u = __ffs(m) - 1;
-                            m &= m - 1;
-                            pair(b + u);
-                        }
+                    const uint32_t lc = row_last_chunk(w);
+                    // two chunks at a time
+                    for (uint32_t c = 0; c <= lc; c += 2) {
+                        uint64_t hits = c == 0 ? (uint32_t)w : more[chunk_at(cap, c, row, t)];
+                        if (c < lc) hits |= (uint64_t)more[chunk_at(cap, c + 1, row, t)] << 32;
+                        pairs((int)(row_first(w) + 32u * c), hits);
                     }
-                } else {
-                    int b, e;
-                    sub_row_slots(srange, S, sub_rows(S, xi), row / 3, row % 3, xi, b, e);
-                    for (int q = b; q < e; ++q)
-                        if (near(q)) pair(q);
+                    continue;
+                }
+                int b, e;
+                sub_row_slots(srange, S, sub_rows(S, xi), row / 3, row % 3, xi, b, e);
+                for (int base = b; base < e; base += 64) {
+                    const int left = min(64, e - base);
+                    uint64_t hits = 0;
+#pragma unroll 4
+                    for (int k = 0; k < left; ++k) {
+                        const float4 xj = spos_s[base + k];
+                        const float dx = xi.x - xj.x, dy = xi.y - xj.y, dz = xi.z - xj.z;
+                        const float r2 = dx * dx + dy * dy + dz * dz;
+                        hits |= (uint64_t)(r2 <= h2 && r2 > 0.0f) << k;
+                    }
+                    pairs(base, hits);
                 }
             }
         }
