@@ -761,7 +761,7 @@ sph_status Engine::autotune(int reps, sph_tuning* out) {
     };
     static const int cand[] = {1, 2, 4, 8, 16};
     static const int caps[] = {32, 40, 48, 64};
-    static const int blks[] = {256, 128};
+    static const int blks[] = {128, 256};
     // without masks: a pass's time with L lanes does not depend on the other's
     float td[17], tf[17];
     for (int L : cand) {
