@@ -315,14 +315,15 @@ const char* sph_last_error_message(const sph_handle* h);
 sph_status sph_enable_timing(sph_handle* h, int32_t enable);
 sph_status sph_stage_times(sph_handle* h, float* ms, int32_t* count);
 const char* sph_stage_name(int32_t stage);
-/* Device time of n steps measured with HIP events recorded on the handle's
- * stream around the steps (no host work inside the timed region). */
-/* Replays the steady-state plain step from captured hipGraphs of one, two and
- * four steps (each captured when a call first has steps for it, re-captured
- * after any change of parameters, kernel variants or learned boundary); steps
- * with per-stage timing on and two-scale steps run eagerly.  No reference counterpart (the reference
+/* Replays the steady-state plain step from captured hipGraphs, at first of one
+ * step, of two and four steps for a call with 16 steps or more left and once
+ * calls have replayed four steps (captured again after any change of
+ * parameters, kernel variants or learned boundary); steps with per-stage timing
+ * on and two-scale steps run eagerly.  No reference counterpart (the reference
  * launches every kernel of every step); as sph_batch_use_graph. */
 sph_status sph_use_graph(sph_handle* h, int32_t enable);
+/* Device time of n steps measured with HIP events recorded on the handle's
+ * stream around the steps (no host work inside the timed region). */
 sph_status sph_time_steps(sph_handle* h, int32_t n_steps, int32_t two_scale,
                           float* ms);
 /* ---- kernel tuning -----------------------------------------------------
@@ -338,7 +339,12 @@ sph_status sph_time_steps(sph_handle* h, int32_t n_steps, int32_t two_scale,
  * the lanes fields are then unused.  One lane per particle in both passes
  * (the default) records them too, with the sums of the loops without masks, in
  * plain steps of one scene of more than 28,672 particles, if the memory is at
- * most an eighth of what is free.  No reference counterpart: the reference
+ * most an eighth of what is free; a handle holds that memory from its creation
+ * until other variants are set or a two-scale step runs, and again from the
+ * next step that reads it.  Sets of up to 28,672 particles with masks, 40,960
+ * with one lane per particle, run sixteen lanes per particle with the same
+ * results, whatever hit_list and block are (two-scale steps with masks do not).
+ * No reference counterpart: the reference
  * fixes one thread per particle and a block size of 256
  * (particle_simulation.cu:1385-1556, 2943-2957); these generalise its launch
  * configuration. */
@@ -353,9 +359,9 @@ typedef struct sph_tuning {
 } sph_tuning;
 sph_status sph_set_tuning(sph_handle* h, const sph_tuning* t);
 sph_status sph_get_tuning(const sph_handle* h, sph_tuning* out);
-/* Times every variant on the current state (needs one step first; each
- * kernel reps times), keeps the fastest, re-runs the last step's density and
- * force with it; out may be NULL. */
+/* Times every variant on the current state as a step like the last one would
+ * run it (needs one step first; each kernel reps times), keeps the fastest,
+ * re-runs the last step's density and force with it; out may be NULL. */
 sph_status sph_autotune(sph_handle* h, int32_t reps, sph_tuning* out);
 /* Re-runs sph_autotune (reps 2) before every steps-th step of sph_step and
  * sph_step_two_scale, on the live state; 0 (the default) turns it off.  The
