@@ -666,15 +666,17 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(8, 8))) void 
                 // a lane without a run reads nothing; its place is any
                 m = density_row<PLAIN>(WindowRow{win + __umul24(b - lo, 3)}, cnt, xi, h2, self, sum, put);
                 wave_sync();   // the next row's window replaces this one
-            } else if (PLAIN && __all(cnt == 0 || cnt > kRowMaxCands)) {
-                // no bits wanted: k_density's loop
-#pragma unroll 4
-                for (int q = (int)b; q < (int)b + cnt; ++q) {
-                    const float d = density_gap(xi, pos[q], h2);
-                    sum += d * d * d;
-                }
             } else if (some) {
-                m = density_row<PLAIN>(GlobalRow{pb, b}, cnt, xi, h2, self, sum, put);
+                if (PLAIN && __all(cnt == 0 || cnt > kRowMaxCands)) {
+                    // no bits wanted: k_density's loop
+#pragma unroll 4
+                    for (int q = (int)b; q < (int)b + cnt; ++q) {
+                        const float d = density_gap(xi, pos[q], h2);
+                        sum += d * d * d;
+                    }
+                } else {
+                    m = density_row<PLAIN>(GlobalRow{pb, b}, cnt, xi, h2, self, sum, put);
+                }
             }
             const uint64_t w = (uint64_t)b << 32 | m;
             if (live)
